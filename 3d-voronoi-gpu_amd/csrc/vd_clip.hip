@@ -916,13 +916,18 @@ __device__ __forceinline__ void accumulate<1>(const ClipArgs& a, int site, const
   atomicAdd(p + 3, (unsigned long long)__double2ll_rn(S.z * kFixScale));
 }
 
+// Adds n pairs to the counter of a status, in the workgroup's set.
+__device__ __forceinline__ void add_status(const ClipArgs& a, int status, unsigned n) {
+  atomicAdd(a.status_hist + (blockIdx.x % kHistStripes) * kHistStride + status, (unsigned long long)n);
+}
+
 __device__ __forceinline__ void count_status(const ClipArgs& a, int status, bool live) {
   if (!a.status_hist) return;
   const int lane = threadIdx.x & 63;
 #pragma unroll
   for (int s = 0; s < 7; ++s) {
     const unsigned long long m = __ballot(live && status == s);
-    if (lane == 0 && m) atomicAdd(a.status_hist + s, (unsigned long long)__popcll(m));
+    if (lane == 0 && m) add_status(a, s, (unsigned)__popcll(m));
   }
 }
 
@@ -1598,7 +1603,7 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
     for (unsigned r = rec_next1 + lane; r < rec_end1 && r < a.rec_cap; r += 64) a.rec_meta[r] = make_uint4(~0u, 0u, 0u, 0u);
   }
   __syncthreads();
-  if (a.status_hist && lane < 7 && hist[lane]) atomicAdd(a.status_hist + lane, (unsigned long long)hist[lane]);
+  if (a.status_hist && lane < 7 && hist[lane]) add_status(a, lane, hist[lane]);
 }
 
 // Emptiness test of the site-major form as a pass of its own, before the
@@ -1747,7 +1752,7 @@ __global__ __launch_bounds__(64) void k_cull_site(ClipArgs a, int depth, unsigne
     }
     if (lane == 0) pair_count[s] = w - pb;
   }
-  if (lane == 0 && a.status_hist && n_culled) atomicAdd(a.status_hist + kNoIntersection, (unsigned long long)n_culled);
+  if (lane == 0 && a.status_hist && n_culled) add_status(a, kNoIntersection, n_culled);
 }
 
 // Volume pass of the site-major form: one lane per record.  The planes are
@@ -1951,8 +1956,7 @@ __global__ __launch_bounds__(kMomentsBlock) void k_site_moments(ClipArgs a) {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
   }
   __syncthreads();
-  if (a.status_hist && threadIdx.x < 7 && hist[threadIdx.x])
-    atomicAdd(a.status_hist + threadIdx.x, (unsigned long long)hist[threadIdx.x]);
+  if (a.status_hist && threadIdx.x < 7 && hist[threadIdx.x]) add_status(a, threadIdx.x, hist[threadIdx.x]);
 }
 
 // ----------------------------------------------------- cell -> tet form ----
@@ -2175,7 +2179,7 @@ __global__ __launch_bounds__(64) void k_cells_clip(ClipArgs a, CellStore cs, int
         }
       }
       count_status(a, cst, false);
-      if (a.status_hist && lane == 0) atomicAdd(a.status_hist + cst, (unsigned long long)(pe - pb));
+      if (a.status_hist && lane == 0) add_status(a, cst, pe - pb);
       continue;
     }
     // the other slot takes this site's cell once no queued pair refers to it

@@ -63,8 +63,16 @@ struct ClipArgs {
   unsigned long long* acc_fix;  // n_sites x 4, 2^-20 fixed point of FP64 pair sums
   uint8_t* pair_status;      // optional, n_pairs
   double* pair_vals;         // optional, n_pairs x 4
-  unsigned long long* status_hist;  // optional, 7 counters
+  unsigned long long* status_hist;  // optional, kHistWords words: kHistStripes sets of 7 counters
 };
+
+// The status counters are kept in kHistStripes sets, each in a cache line of
+// its own; a workgroup adds to set blockIdx % kHistStripes and the reader sums
+// the sets.  Atomics on one address complete one after another at 13 ns each
+// (the emptiness pass took 190 us for 14,633 workgroups and 445 us for 32,768
+// whatever its pairs were, with one set).
+constexpr int kHistStripes = 64, kHistStride = 16;
+constexpr int kHistWords = kHistStripes * kHistStride;
 
 // Cells of kernel B, kept for kernel C: per site its status, plane and
 // triangle counts, squared radius of its farthest vertex, planes [pcap] and

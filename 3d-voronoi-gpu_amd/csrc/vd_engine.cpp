@@ -419,7 +419,7 @@ int vd_ctx_create(vd_ctx** out, int device, const vd_config* cfg) {
   }
   for (auto& row : ctx->ev)
     for (auto& e : row) (void)hipEventCreate(&e);
-  if (ensure_offsets(ctx) != VD_OK || ctx->hist.ensure(8) != hipSuccess) {
+  if (ensure_offsets(ctx) != VD_OK || ctx->hist.ensure(vd::kHistWords) != hipSuccess) {
     fprintf(stderr, "vd_ctx_create: %s\n", ctx->err.c_str());
     vd_ctx_destroy(ctx);
     return VD_ERR_HIP;
@@ -749,7 +749,7 @@ int vd_clip_step(vd_ctx* ctx) {
     VD_HIP(ctx->acc_fix.ensure(4 * (size_t)n), "alloc acc");
     VD_HIP(vd::fill_u32(ctx->acc_fix.p, 8LL * n, 0u, ctx->stream), "clear acc");
   }
-  VD_HIP(vd::fill_u32(ctx->hist.p, 16, 0u, ctx->stream), "clear hist");
+  VD_HIP(vd::fill_u32(ctx->hist.p, 2 * vd::kHistWords, 0u, ctx->stream), "clear hist");
   if (c.record_pairs) {
     VD_HIP(ctx->pair_status.ensure(std::max(n_pairs, 1LL)), "alloc pair status");
     VD_HIP(ctx->pair_vals.ensure(4 * std::max(n_pairs, 1LL)), "alloc pair vals");
@@ -1360,10 +1360,13 @@ int vd_get_tet_knn_range(vd_ctx* ctx, int first_tet, int n_tets, int32_t* out) {
 
 int vd_get_status_hist(vd_ctx* ctx, uint64_t* hist7) {
   if (!ctx || !hist7) return VD_ERR_ARG;
-  unsigned long long h[8];
+  unsigned long long h[vd::kHistWords];
   VD_HIP(hipMemcpyAsync(h, ctx->hist.p, sizeof h, hipMemcpyDeviceToHost, ctx->stream), "read hist");
   VD_HIP(hipStreamSynchronize(ctx->stream), "read hist");
-  for (int i = 0; i < 7; ++i) hist7[i] = h[i];
+  for (int i = 0; i < 7; ++i) {
+    hist7[i] = 0;
+    for (int s = 0; s < vd::kHistStripes; ++s) hist7[i] += h[s * vd::kHistStride + i];
+  }
   return VD_OK;
 }
 
