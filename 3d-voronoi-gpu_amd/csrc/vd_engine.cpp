@@ -326,6 +326,7 @@ vd::GridBufs grid_bufs(vd_ctx* ctx) {
     gb.pt_begin = ctx->b_site_begin.p;
     gb.pt_inst = ctx->b_site_inst.p;
     gb.box = ctx->b_box.p;
+    for (const auto& q : ctx->inst) gb.max_pts = std::max(gb.max_pts, q.ns);
   }
   gb.max_cells = ctx->max_cells;
   gb.count = ctx->g_count.p;

@@ -24,6 +24,7 @@
 #include "vd_knn.hpp"
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <vector>
 
@@ -131,23 +132,8 @@ __device__ __forceinline__ float dist2(const float4& r, const float4& q) {
 
 // ---------------------------------------------------------------- grid ----
 
-// Bounding box of the points (and of `extra`, a box given by the host), then
-// the grid shape: about n/density cells of equal size, at most max_cells.
-// One block per instance.
-__global__ __launch_bounds__(kScanThreads) void k_grid_shape(const float4* pts, int n, const int* pt_begin,
-                                                              const int* cell_base, const float* box, float3 extra_lo,
-                                                              float3 extra_hi, int use_extra, float density,
-                                                              int max_cells, GridShape* shapes) {
-  __shared__ float red[6][kScanThreads / 64];
-  const int inst = blockIdx.x;
-  const int p0 = pt_begin ? pt_begin[inst] : 0, p1 = pt_begin ? pt_begin[inst + 1] : n;
-  if (cell_base) max_cells = cell_base[inst + 1] - cell_base[inst];
-  if (box) {
-    extra_lo = make_float3(box[6 * inst], box[6 * inst + 1], box[6 * inst + 2]);
-    extra_hi = make_float3(box[6 * inst + 3], box[6 * inst + 4], box[6 * inst + 5]);
-    use_extra = 1;
-  }
-  n = p1 - p0;
+// Bounding box of points p0..p1 over the workgroup, a part per wave in red.
+__device__ __forceinline__ void points_box(const float4* pts, int p0, int p1, float (*red)[kScanThreads / 64]) {
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int i = p0 + threadIdx.x; i < p1; i += blockDim.x) {
     const float4 p = pts[i];
@@ -159,63 +145,128 @@ __global__ __launch_bounds__(kScanThreads) void k_grid_shape(const float4* pts, 
       lo[a] = fminf(lo[a], __shfl_xor(lo[a], off));
       hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], off));
     }
-  const int w = threadIdx.x >> 6;
   if ((threadIdx.x & 63) == 0)
     for (int a = 0; a < 3; ++a) {
-      red[a][w] = lo[a];
-      red[3 + a][w] = hi[a];
+      red[a][threadIdx.x >> 6] = lo[a];
+      red[3 + a][threadIdx.x >> 6] = hi[a];
     }
   __syncthreads();
+}
+__device__ __forceinline__ void join_boxes(float (*red)[kScanThreads / 64], float lo[3], float hi[3]) {
+  for (int a = 0; a < 3; ++a) {
+    lo[a] = red[a][0];
+    hi[a] = red[3 + a][0];
+    for (int j = 1; j < (int)(blockDim.x >> 6); ++j) {
+      lo[a] = fminf(lo[a], red[a][j]);
+      hi[a] = fmaxf(hi[a], red[3 + a][j]);
+    }
+  }
+}
+
+// Grid shape of n points with bounding box lo..hi, which it extends by the box
+// extra_lo..extra_hi (use_extra): about n/density cells of equal size, at most
+// max_cells.
+__device__ GridShape make_shape(const float lo[3], const float hi[3], const float3& extra_lo, const float3& extra_hi,
+                                int use_extra, int n, float density, int max_cells) {
+  double l[3], h[3];
+  const float elo[3] = {extra_lo.x, extra_lo.y, extra_lo.z}, ehi[3] = {extra_hi.x, extra_hi.y, extra_hi.z};
+  for (int a = 0; a < 3; ++a) {
+    l[a] = lo[a];
+    h[a] = hi[a];
+    if (use_extra) {
+      l[a] = fmin(l[a], (double)elo[a]);
+      h[a] = fmax(h[a], (double)ehi[a]);
+    }
+    if (!(l[a] <= h[a])) { l[a] = 0.0; h[a] = 0.0; }
+  }
+  double ext = fmax(fmax(h[0] - l[0], h[1] - l[1]), fmax(h[2] - l[2], 1e-20));
+  // pad the box so that no point sits on the upper face
+  for (int a = 0; a < 3; ++a) {
+    l[a] -= 1e-4 * ext;
+    h[a] += 1e-4 * ext;
+  }
+  ext *= 1.0002;
+  double vol = 1.0;
+  for (int a = 0; a < 3; ++a) vol *= fmax(h[a] - l[a], ext * 1e-3);
+  const double cells = fmax(1.0, (double)n / (double)density);
+  double cs = cbrt(vol / cells);
+  int dim[3];
+  for (;;) {
+    long long tot = 1;
+    for (int a = 0; a < 3; ++a) {
+      dim[a] = (int)fmin(1024.0, fmax(1.0, ceil((h[a] - l[a]) / cs)));
+      tot *= dim[a];
+    }
+    if (tot <= max_cells) break;
+    cs *= 1.05;
+  }
+  GridShape g;
+  for (int a = 0; a < 3; ++a) {
+    g.lo[a] = (float)l[a];
+    g.dim[a] = dim[a];
+  }
+  g.h = (float)cs;
+  g.inv_h = (float)(1.0 / cs);
+  g.ncell = dim[0] * dim[1] * dim[2];
+  // absolute slack for the cell-box distance bounds (rounding of the cell
+  // assignment and of lo + c*h)
+  g.slack = (float)(1e-3 * cs + 1e-6 * (fabs(l[0]) + fabs(l[1]) + fabs(l[2]) + 1024.0 * cs));
+  return g;
+}
+
+// Bounding boxes of the n points' parts, one workgroup each, for
+// k_grid_shape's `parts` (6 floats per workgroup).
+constexpr int kBoxParts = 64;
+__global__ __launch_bounds__(kScanThreads) void k_grid_box(const float4* pts, int n, float* parts) {
+  __shared__ float red[6][kScanThreads / 64];
+  const int per = (n + (int)gridDim.x - 1) / (int)gridDim.x;
+  const int p0 = min(n, (int)blockIdx.x * per);
+  points_box(pts, p0, min(n, p0 + per), red);
   if (threadIdx.x == 0) {
-    for (int j = 1; j < (int)(blockDim.x >> 6); ++j)
-      for (int a = 0; a < 3; ++a) {
-        red[a][0] = fminf(red[a][0], red[a][j]);
-        red[3 + a][0] = fmaxf(red[3 + a][0], red[3 + a][j]);
-      }
-    double l[3], h[3];
-    const float elo[3] = {extra_lo.x, extra_lo.y, extra_lo.z}, ehi[3] = {extra_hi.x, extra_hi.y, extra_hi.z};
+    float lo[3], hi[3];
+    join_boxes(red, lo, hi);
     for (int a = 0; a < 3; ++a) {
-      l[a] = red[a][0];
-      h[a] = red[3 + a][0];
-      if (use_extra) {
-        l[a] = fmin(l[a], (double)elo[a]);
-        h[a] = fmax(h[a], (double)ehi[a]);
-      }
-      if (!(l[a] <= h[a])) { l[a] = 0.0; h[a] = 0.0; }
+      parts[6 * blockIdx.x + a] = lo[a];
+      parts[6 * blockIdx.x + 3 + a] = hi[a];
     }
-    double ext = fmax(fmax(h[0] - l[0], h[1] - l[1]), fmax(h[2] - l[2], 1e-20));
-    // pad the box so that no point sits on the upper face
+  }
+}
+
+// The grid shape over the points' bounding box (and `extra`, a box given by
+// the host); one block per instance.  The single instance may give the boxes
+// of its points' parts (k_grid_box) instead of having one workgroup read all
+// points (100,000: 41 us -> 11 for both kernels; 200,000: 90 -> 11).
+__global__ __launch_bounds__(kScanThreads) void k_grid_shape(const float4* pts, int n, const int* pt_begin,
+                                                              const int* cell_base, const float* box, float3 extra_lo,
+                                                              float3 extra_hi, int use_extra, float density,
+                                                              int max_cells, const float* parts, int n_parts,
+                                                              GridShape* shapes) {
+  __shared__ float red[6][kScanThreads / 64];
+  const int inst = blockIdx.x;
+  const int p0 = pt_begin ? pt_begin[inst] : 0, p1 = pt_begin ? pt_begin[inst + 1] : n;
+  if (cell_base) max_cells = cell_base[inst + 1] - cell_base[inst];
+  if (box) {
+    extra_lo = make_float3(box[6 * inst], box[6 * inst + 1], box[6 * inst + 2]);
+    extra_hi = make_float3(box[6 * inst + 3], box[6 * inst + 4], box[6 * inst + 5]);
+    use_extra = 1;
+  }
+  float lo[3], hi[3];
+  if (parts) {  // one wave
+    const int lane = threadIdx.x;
     for (int a = 0; a < 3; ++a) {
-      l[a] -= 1e-4 * ext;
-      h[a] += 1e-4 * ext;
-    }
-    ext *= 1.0002;
-    double vol = 1.0;
-    for (int a = 0; a < 3; ++a) vol *= fmax(h[a] - l[a], ext * 1e-3);
-    const double cells = fmax(1.0, (double)n / (double)density);
-    double cs = cbrt(vol / cells);
-    int dim[3];
-    for (;;) {
-      long long tot = 1;
-      for (int a = 0; a < 3; ++a) {
-        dim[a] = (int)fmin(1024.0, fmax(1.0, ceil((h[a] - l[a]) / cs)));
-        tot *= dim[a];
+      lo[a] = lane < n_parts ? parts[6 * lane + a] : INFINITY;
+      hi[a] = lane < n_parts ? parts[6 * lane + 3 + a] : -INFINITY;
+      for (int off = 32; off > 0; off >>= 1) {
+        lo[a] = fminf(lo[a], __shfl_xor(lo[a], off));
+        hi[a] = fmaxf(hi[a], __shfl_xor(hi[a], off));
       }
-      if (tot <= max_cells) break;
-      cs *= 1.05;
     }
-    GridShape g;
-    for (int a = 0; a < 3; ++a) {
-      g.lo[a] = (float)l[a];
-      g.dim[a] = dim[a];
-    }
-    g.h = (float)cs;
-    g.inv_h = (float)(1.0 / cs);
-    g.ncell = dim[0] * dim[1] * dim[2];
-    // absolute slack for the cell-box distance bounds (rounding of the cell
-    // assignment and of lo + c*h)
-    g.slack = (float)(1e-3 * cs + 1e-6 * (fabs(l[0]) + fabs(l[1]) + fabs(l[2]) + 1024.0 * cs));
-    shapes[inst] = g;
+  } else {
+    points_box(pts, p0, p1, red);
+  }
+  if (threadIdx.x == 0) {
+    if (!parts) join_boxes(red, lo, hi);
+    shapes[inst] = make_shape(lo, hi, extra_lo, extra_hi, use_extra, p1 - p0, density, max_cells);
   }
 }
 
@@ -241,23 +292,162 @@ __global__ void k_grid_scatter(int n, const int* cell_of, const int* start, int*
   sorted_ids[start[c] + atomicAdd(cursor + c, 1)] = i;
 }
 
-// One thread per cell: order the cell's ids, then gather the points.
+// Orders every cell's points by index: each point's place is the number of
+// smaller ids in its cell, so the loads of a cell do not depend on each other.
+// sorted_pts gets the points (their ids in w) and then sorted_ids the ids.  A
+// workgroup takes kSortCells cells: a lane of its first wave a cell of at most
+// kLightCell points, and the workgroup together each fuller one.  (One lane
+// inserting a cell's ids one by one took 4.3 ms at 200,000 clustered sites,
+// where a cell holds up to a few thousand; one wave per heavy cell 0.45 ms;
+// this 0.11 ms.)
 // n_cells < 0: the cells of the single instance gs[0].
-__global__ void k_grid_sort(const GridShape* gs, int n_cells, const float4* pts, const int* start, int* sorted_ids,
-                            float4* sorted_pts) {
-  const int c = blockIdx.x * blockDim.x + threadIdx.x;
-  if (c >= (n_cells >= 0 ? n_cells : gs->ncell)) return;
-  const int b = start[c], e = start[c + 1];
-  for (int i = b + 1; i < e; ++i) {
-    const int v = sorted_ids[i];
-    int j = i - 1;
-    while (j >= b && sorted_ids[j] > v) {
-      sorted_ids[j + 1] = sorted_ids[j];
-      --j;
+constexpr int kLightCell = 16, kSortCells = 64, kSortThreads = 256, kSortTile = 1024;
+__device__ __forceinline__ float4 with_id(float4 p, int id) {
+  p.w = __int_as_float(id);
+  return p;
+}
+__global__ __launch_bounds__(kSortThreads) void k_grid_sort(const GridShape* gs, int n_cells, const float4* pts,
+                                                            const int* start, int* sorted_ids, float4* sorted_pts) {
+  __shared__ int4 tile[kSortTile / 4];
+  __shared__ int heavy_b[kSortCells], heavy_e[kSortCells];
+  __shared__ int n_heavy;
+  const int tid = threadIdx.x;
+  int b = 0, e = 0;
+  if (tid < kSortCells) {
+    const int c = blockIdx.x * kSortCells + tid;
+    if (c < (n_cells >= 0 ? n_cells : gs->ncell)) {
+      b = start[c];
+      e = start[c + 1];
     }
-    sorted_ids[j + 1] = v;
+    const bool heavy = e - b > kLightCell;
+    const uint64_t m = __ballot(heavy);
+    if (heavy) {
+      const int k = __popcll(m & ((1ull << tid) - 1ull));
+      heavy_b[k] = b;
+      heavy_e[k] = e;
+      b = e;
+    }
+    if (tid == 0) n_heavy = __popcll(m);
+    for (int i = b; i < e; ++i) {
+      const int v = sorted_ids[i];
+      int rank = 0;
+      for (int j = b; j < e; ++j) rank += sorted_ids[j] < v;
+      sorted_pts[b + rank] = with_id(pts[v], v);
+    }
   }
-  for (int i = b; i < e; ++i) sorted_pts[i] = pts[sorted_ids[i]];
+  __syncthreads();
+  for (int h = 0; h < n_heavy; ++h) {
+    const int hb = heavy_b[h], he = heavy_e[h];
+    for (int i0 = hb; i0 < he; i0 += kSortThreads) {
+      const int i = i0 + tid;
+      const int v = i < he ? sorted_ids[i] : INT_MAX;
+      int rank = 0;
+      for (int t0 = hb; t0 < he; t0 += kSortTile) {
+        __syncthreads();
+        for (int j = tid; j < kSortTile; j += kSortThreads)
+          ((int*)tile)[j] = t0 + j < he ? sorted_ids[t0 + j] : INT_MAX;
+        __syncthreads();
+        const int n4 = (min(kSortTile, he - t0) + 3) / 4;
+        for (int j = 0; j < n4; ++j) {
+          const int4 q = tile[j];
+          rank += (q.x < v) + (q.y < v) + (q.z < v) + (q.w < v);
+        }
+      }
+      if (i < he) sorted_pts[hb + rank] = with_id(pts[v], v);
+    }
+  }
+  __threadfence_block();
+  __syncthreads();
+  if (tid < kSortCells)
+    for (int i = b; i < e; ++i) sorted_ids[i] = __float_as_int(sorted_pts[i].w);
+  for (int h = 0; h < n_heavy; ++h)
+    for (int i = heavy_b[h] + tid; i < heavy_e[h]; i += kSortThreads) sorted_ids[i] = __float_as_int(sorted_pts[i].w);
+}
+
+// The whole grid build of an instance of at most kSmallPoints points and
+// kSmallCells cells in one workgroup, with the cell counts and the ids in LDS:
+// box and shape, counts, scan, scatter, order in the cells.  One launch
+// instead of eight, whose latencies are all that small problems pay (1,037
+// points: 43 us -> 9.3; 131: 42 -> 7.6).  The limit is what the LDS holds with
+// room to spare; at 3,001 points the one workgroup takes 17 us (the eight
+// launches 43).  The tables are those of the other path.
+constexpr int kSmallPoints = 8192, kSmallCells = 8192;
+__global__ __launch_bounds__(kScanThreads) void k_grid_small(const float4* pts, int n, const int* pt_begin,
+                                                              const int* cell_base, const float* box, float3 extra_lo,
+                                                              float3 extra_hi, int use_extra, float density,
+                                                              int max_cells, int n_inst, GridShape* shapes, int* count,
+                                                              int* start, int* sorted_ids, float4* sorted_pts) {
+  __shared__ float red[6][kScanThreads / 64];
+  __shared__ int wsum[kScanThreads / 64];
+  __shared__ GridShape g;
+  __shared__ int cnt[kSmallCells];
+  __shared__ int ids[kSmallPoints];
+  const int inst = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int p0 = pt_begin ? pt_begin[inst] : 0, p1 = pt_begin ? pt_begin[inst + 1] : n;
+  const int c0 = cell_base ? cell_base[inst] : 0;
+  const int cells = (cell_base ? cell_base[inst + 1] : max_cells) - c0;
+  const int np = p1 - p0;
+  if (box) {
+    extra_lo = make_float3(box[6 * inst], box[6 * inst + 1], box[6 * inst + 2]);
+    extra_hi = make_float3(box[6 * inst + 3], box[6 * inst + 4], box[6 * inst + 5]);
+    use_extra = 1;
+  }
+  points_box(pts, p0, p1, red);
+  if (tid == 0) {
+    float lo[3], hi[3];
+    join_boxes(red, lo, hi);
+    g = make_shape(lo, hi, extra_lo, extra_hi, use_extra, np, density, cells);
+    shapes[inst] = g;
+  }
+  for (int i = tid; i < cells; i += kScanThreads) cnt[i] = 0;
+  __syncthreads();
+  auto cell_at = [&](const float4& p) {
+    const int cx = cell_coord(p.x, g.lo[0], g.inv_h, g.dim[0]);
+    const int cy = cell_coord(p.y, g.lo[1], g.inv_h, g.dim[1]);
+    const int cz = cell_coord(p.z, g.lo[2], g.inv_h, g.dim[2]);
+    return cx + g.dim[0] * (cy + g.dim[1] * cz);
+  };
+  for (int i = tid; i < np; i += kScanThreads) atomicAdd(&cnt[cell_at(pts[p0 + i])], 1);
+  __syncthreads();
+  // exclusive scan of the counts, kPer consecutive cells per thread
+  constexpr int kPer = kSmallCells / kScanThreads;
+  int v[kPer], sum = 0;
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int c = tid * kPer + k;
+    v[k] = c < cells ? cnt[c] : 0;
+    sum += v[k];
+  }
+  const int incl = wave_incl_sum(sum);
+  if (lane == 63) wsum[wv] = incl;
+  __syncthreads();
+  int run = incl - sum;
+  for (int w = 0; w < wv; ++w) run += wsum[w];
+#pragma unroll
+  for (int k = 0; k < kPer; ++k) {
+    const int c = tid * kPer + k;
+    if (c < cells) {
+      count[c0 + c] = v[k];
+      start[c0 + c] = p0 + run;
+      cnt[c] = run;
+    }
+    run += v[k];
+  }
+  if (inst == n_inst - 1 && tid == 0) start[c0 + cells] = p1;
+  __syncthreads();
+  for (int i = tid; i < np; i += kScanThreads) ids[atomicAdd(&cnt[cell_at(pts[p0 + i])], 1)] = p0 + i;
+  __syncthreads();
+  // cnt[c] is now the end of cell c, so its start is the end of cell c - 1
+  for (int i = tid; i < np; i += kScanThreads) {
+    const int id = ids[i];
+    const float4 p = pts[id];
+    const int c = cell_at(p);
+    const int b = c > 0 ? cnt[c - 1] : 0, e = cnt[c];
+    int rank = 0;
+    for (int j = b; j < e; ++j) rank += ids[j] < id;
+    sorted_ids[p0 + b + rank] = id;
+    sorted_pts[p0 + b + rank] = with_id(p, id);
+  }
 }
 
 // ---------------------------------------------------------------- query ---
@@ -557,7 +747,6 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
         if (f < total) {
           const int idx = o_st + (f - o_ex);
           p = a.sorted_pts[idx];
-          p.w = __uint_as_float((uint32_t)a.sorted_ids[idx]);
           keep = !(dist2(p, c) > R2);
         }
         const uint64_t m = __ballot(keep);
@@ -734,8 +923,9 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       bool ok = false;
       if (f < total) {
         const int idx = o_st + (f - o_ex);
-        const int id = a.sorted_ids[idx];
-        key = knn_key(dist2(a.sorted_pts[idx], qp), (uint32_t)id);
+        const float4 p = a.sorted_pts[idx];
+        const int id = __float_as_int(p.w);
+        key = knn_key(dist2(p, qp), (uint32_t)id);
         ok = (id != self) && key < thr;
       }
       push(key, ok);
@@ -752,7 +942,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       if (f < r1) {
         // skip cells already visited: those inside the offset table's reach
         const float4 p = a.sorted_pts[f];
-        const int id = a.sorted_ids[f];
+        const int id = __float_as_int(p.w);
         const int cx = cell_coord(p.x, g.lo[0], g.inv_h, g.dim[0]) - qc[0];
         const int cy = cell_coord(p.y, g.lo[1], g.inv_h, g.dim[1]) - qc[1];
         const int cz = cell_coord(p.z, g.lo[2], g.inv_h, g.dim[2]) - qc[2];
@@ -876,6 +1066,7 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const int* in, const int* n
   const int n = scan_n(n_dev, n_max);
   const long long base = (long long)blockIdx.x * kScanTile;
   if (base >= n && blockIdx.x > 0) return;
+  const bool only = n_max <= kScanTile;  // the tile is the whole scan
   T v[kScanItems];
   T s = 0;
 #pragma unroll
@@ -916,7 +1107,12 @@ __global__ __launch_bounds__(1024) void k_scan_tiles(const int* in, const int* n
       if (cursor) cursor[i] = 0;
     }
   }
-  if (threadIdx.x == 1023) tile_sum[blockIdx.x] = part[1023];
+  if (threadIdx.x == 1023) {
+    if (only)
+      out[n] = part[1023];
+    else
+      tile_sum[blockIdx.x] = part[1023];
+  }
 }
 
 template <class T>
@@ -960,6 +1156,7 @@ static hipError_t scan_excl_t(const int* in, const int* n_dev, int n_max, T* out
                               hipStream_t st) {
   const int tiles = std::max(1, (n_max + kScanTile - 1) / kScanTile);
   hipLaunchKernelGGL(k_scan_tiles<T>, dim3(tiles), dim3(1024), 0, st, in, n_dev, n_max, out, cursor, tmp);
+  if (n_max <= kScanTile) return hipGetLastError();
   hipLaunchKernelGGL(k_scan_top<T>, dim3(1), dim3(1024), 0, st, n_dev, n_max, tmp);
   hipLaunchKernelGGL(k_scan_add<T>, dim3((unsigned)(((long long)n_max + 1 + 255) / 256)), dim3(256), 0, st, n_dev,
                      n_max, out, tmp);
@@ -1001,8 +1198,21 @@ hipError_t grid_build(const GridBufs& gb, const float4* pts, int n, const float*
   const float3 elo = extra_lo ? make_float3(extra_lo[0], extra_lo[1], extra_lo[2]) : make_float3(0, 0, 0);
   const float3 ehi = extra_hi ? make_float3(extra_hi[0], extra_hi[1], extra_hi[2]) : make_float3(0, 0, 0);
   if (gb.n_inst < 1 || (gb.n_inst > 1 && (!gb.cell_base || !gb.pt_begin || !gb.pt_inst))) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_grid_shape, dim3((unsigned)gb.n_inst), dim3(kScanThreads), 0, st, pts, n, gb.pt_begin,
-                     gb.cell_base, gb.box, elo, ehi, extra_lo ? 1 : 0, density, gb.max_cells, gb.shape);
+  const int max_pts = gb.n_inst == 1 ? n : gb.max_pts;
+  if (max_pts > 0 && max_pts <= kSmallPoints &&
+      (gb.n_inst == 1 ? gb.max_cells : grid_max_cells(max_pts, density)) <= kSmallCells) {
+    hipLaunchKernelGGL(k_grid_small, dim3((unsigned)gb.n_inst), dim3(kScanThreads), 0, st, pts, n, gb.pt_begin,
+                       gb.cell_base, gb.box, elo, ehi, extra_lo ? 1 : 0, density, gb.max_cells, gb.n_inst, gb.shape,
+                       gb.count, gb.start, gb.sorted_ids, gb.sorted_pts);
+    return hipGetLastError();
+  }
+  // the parts' boxes in the count table, which is cleared after the shape
+  const bool parts = gb.n_inst == 1 && !gb.pt_begin && n > kSmallPoints && gb.max_cells >= 6 * kBoxParts;
+  if (parts)
+    hipLaunchKernelGGL(k_grid_box, dim3(kBoxParts), dim3(kScanThreads), 0, st, pts, n, (float*)gb.count);
+  hipLaunchKernelGGL(k_grid_shape, dim3((unsigned)gb.n_inst), dim3(parts ? 64 : kScanThreads), 0, st, pts, n,
+                     gb.pt_begin, gb.cell_base, gb.box, elo, ehi, extra_lo ? 1 : 0, density, gb.max_cells,
+                     parts ? (const float*)gb.count : nullptr, kBoxParts, gb.shape);
   hipError_t e = fill_u32(gb.count, gb.max_cells, 0u, st);
   if (e != hipSuccess) return e;
   const int nb = (n + 255) / 256;
@@ -1017,8 +1227,8 @@ hipError_t grid_build(const GridBufs& gb, const float4* pts, int n, const float*
   if (n > 0)
     hipLaunchKernelGGL(k_grid_scatter, dim3(nb), dim3(256), 0, st, n, gb.cell_of, gb.start, gb.cursor,
                        gb.sorted_ids);
-  hipLaunchKernelGGL(k_grid_sort, dim3((gb.max_cells + 255) / 256), dim3(256), 0, st, gb.shape,
-                     gb.n_inst == 1 ? -1 : gb.max_cells, pts, gb.start, gb.sorted_ids, gb.sorted_pts);
+  hipLaunchKernelGGL(k_grid_sort, dim3((gb.max_cells + kSortCells - 1) / kSortCells), dim3(kSortThreads), 0, st,
+                     gb.shape, gb.n_inst == 1 ? -1 : gb.max_cells, pts, gb.start, gb.sorted_ids, gb.sorted_pts);
   return hipGetLastError();
 }
 

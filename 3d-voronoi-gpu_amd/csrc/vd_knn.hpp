@@ -33,12 +33,13 @@ struct GridBufs {
   const int* pt_inst = nullptr;    // instance of every point, or null
   const float* box = nullptr;      // n_inst x (lo xyz, hi xyz): box the grid must cover besides its points, or null
   int max_cells = 0;               // total cells (cell_base[n_inst])
+  int max_pts = 0;                 // points of the largest instance (0: unknown; one instance: not needed)
   int* count = nullptr;            // max_cells
   int* start = nullptr;            // max_cells + 1
   int* cursor = nullptr;           // max_cells
   int* cell_of = nullptr;          // n
   int* sorted_ids = nullptr;       // n
-  float4* sorted_pts = nullptr;    // n
+  float4* sorted_pts = nullptr;    // n: the points, their ids in w
   int* scan_tmp = nullptr;         // scan_tmp_ints(max_cells)
 };
 
