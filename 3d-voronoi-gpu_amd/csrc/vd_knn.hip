@@ -482,6 +482,7 @@ struct QueryArgs {
   // reference points by original id
   const float4* hint_pts;
   const int* pt_begin;  // first point of every instance (n_inst + 1), or null
+  int run;              // consecutive queries per wave (launch_query)
 };
 
 template <int M>
@@ -629,10 +630,19 @@ constexpr int kQueryWavesDefault = 4;
 // place of one that it excludes, mode 0 and 3), so its k-th key is below that
 // bound (rounded up by a 1e-5 margin) and candidates beyond it are never
 // staged, and the cell walk stops there.
+//
+// Fewer queries than kQueryRun for every wave that the GPU holds at once
+// (kQueryFill) are spread over all of them instead, down to one query per
+// wave, which walks the grid alone (kNN phase at 10,368 tets / 1,037 sites:
+// 115 us in runs of 6 or 5, 79 in runs of 2 and 1; 146,334 tets / 14,633
+// sites: 275 us, 269; the same from 4,096 to 8,192).
 #ifndef VD_KNN_RUN
 #define VD_KNN_RUN 6
 #endif
-constexpr int kQueryRun = VD_KNN_RUN;
+#ifndef VD_KNN_FILL
+#define VD_KNN_FILL 4096
+#endif
+constexpr int kQueryRun = VD_KNN_RUN, kQueryFill = VD_KNN_FILL;
 
 // After the first query of a run, the points that the run's other queries can
 // need are gathered once into LDS (at most kUnionCap): query i's k-th distance
@@ -693,7 +703,8 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
   uint64_t* stage = stage_all[wv];
   int* mark = mark_all[wv];
   float4* uni = uni_all[wv];
-  const int q0 = (blockIdx.x * kQueryWaves + wv) * kQueryRun;
+  const int run = a.run;
+  const int q0 = (blockIdx.x * kQueryWaves + wv) * run;
   int nq = a.n_query;
   if (a.n_query_dev) nq = min(nq, (int)min(*a.n_query_dev, (unsigned)a.n_query));
   float prev_r = -1.f;
@@ -769,8 +780,8 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
   // within max_j(|q_j - c| + r_j) of the centre c of the run's queries (r_j:
   // query j's bound), and every query of the run, the first one included,
   // scans it instead of walking the grid, with the walk's keys and bounds.
-  if (use_hint) {
-    const int n_run = min(q0 + kQueryRun, nq) - q0;
+  if (use_hint && run > 1) {
+    const int n_run = min(q0 + run, nq) - q0;
     float4 pj = {0.f, 0.f, 0.f, 0.f};
     int sj = -1, rj = 0, ij = 0;
     const bool in = lane < n_run;
@@ -812,7 +823,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       }
     }
   }
-  for (int q = q0; q < q0 + kQueryRun && q < nq; ++q) {  // wave-uniform
+  for (int q = q0; q < q0 + run && q < nq; ++q) {  // wave-uniform
 
   float4 qp;
   int self, out_row, inst;
@@ -982,7 +993,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
   prev_qp = qp;
   prev_inst = inst;
 
-  const int q_end = min(q0 + kQueryRun, nq);
+  const int q_end = min(q0 + run, nq);
   if (q == q0 && n_uni < 0 && prev_r >= 0.f && q + 1 < q_end) {
     // the run's other queries: their points (lane j takes query q0 + j)
     float4 pj = qp;
@@ -1235,7 +1246,7 @@ hipError_t grid_build(const GridBufs& gb, const float4* pts, int n, const float*
 namespace {
 template <int W>
 hipError_t launch_query_w(const QueryArgs& a, int n_query, hipStream_t st) {
-  const dim3 grid((n_query + W * kQueryRun - 1) / (W * kQueryRun)), block(64 * W);
+  const dim3 grid((n_query + W * a.run - 1) / (W * a.run)), block(64 * W);
   if (a.k <= 64)
     hipLaunchKernelGGL((k_knn_query<1, W>), grid, block, 0, st, a);
   else if (a.k <= 128)
@@ -1244,7 +1255,8 @@ hipError_t launch_query_w(const QueryArgs& a, int n_query, hipStream_t st) {
     hipLaunchKernelGGL((k_knn_query<4, W>), grid, block, 0, st, a);
   return hipGetLastError();
 }
-hipError_t launch_query(const QueryArgs& a, int n_query, int waves, hipStream_t st) {
+hipError_t launch_query(QueryArgs a, int n_query, int waves, hipStream_t st) {
+  a.run = std::max(1, std::min(kQueryRun, n_query / kQueryFill));
   if (waves == 2) return launch_query_w<2>(a, n_query, st);
   if (waves == 8) return launch_query_w<8>(a, n_query, st);
   return launch_query_w<kQueryWavesDefault>(a, n_query, st);

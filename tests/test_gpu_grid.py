@@ -60,3 +60,23 @@ def test_batch_grids(vdn, O, sizes):
         np.testing.assert_array_equal(sk[off[i]:off[i + 1]] - off[i], O.site_knn(s, 20))
         np.testing.assert_array_equal(tk[t0:t0 + len(t)] - off[i], O.tet_knn(v, t, s, 16))
         t0 += len(t)
+
+
+@pytest.mark.parametrize("n,k", [(4095, 90), (8191, 65), (8192, 20), (8193, 64), (12289, 90), (24577, 20)])
+def test_runs_of_queries(vdn, O, n, k):
+    """Query counts around the multiples of 4,096 at which a wave's run of
+    queries grows from one to six; the second step starts from the first's rows."""
+    from voronoi_amd import meshgen
+
+    verts, tets, sites = meshgen.make_problem("cube", 5, n, seed=70 + n % 10)
+    with vdn.Engine(tet_k=16, site_k=k, accum="f64") as e:
+        e.set_mesh(verts, tets)
+        e.set_sites(sites)
+        for step in range(4):
+            cur = e.sites()
+            e.knn_step()
+            print(f"{n} step {step}", flush=True)
+            np.testing.assert_array_equal(e.site_knn(), O.site_knn(cur, k))
+            np.testing.assert_array_equal(e.tet_knn(), O.tet_knn(verts, tets, cur, 16))
+            e.clip_step()
+            e.update_step()
