@@ -172,17 +172,20 @@ struct vd_ctx {
   DevBuf<double> moments;
   DevBuf<uint8_t> pair_status;
   DevBuf<double> pair_vals;
+  // the status counters (vd::kHistWords) and then the step's other counters,
+  // each in a cache line of its own, cleared together
   DevBuf<unsigned long long> hist;
+  enum Counter { kSiteCounter, kRetryCount, kRetryCount2, kRecCount, kSrnrCount, kCounters };
+  static constexpr int kCounterStride = 32;
+  static constexpr int kCounterWords = 2 * vd::kHistWords + kCounters * kCounterStride;
+  unsigned* counter(Counter c) { return (unsigned*)hist.p + 2 * vd::kHistWords + c * kCounterStride; }
   DevBuf<unsigned> retry_list;
-  DevBuf<unsigned> retry_count;
-  DevBuf<unsigned> retry_list2, retry_count2;  // overflows of the first re-clip
-  DevBuf<unsigned> site_counter;
+  DevBuf<unsigned> retry_list2;  // overflows of the first re-clip
   // site-major form: records of finished polytopes for the volume pass
   DevBuf<uint4> rec_meta;
   DevBuf<uint32_t> rec_tris;
-  DevBuf<unsigned> rec_count;
   // pairs retried with deeper neighbour lists (srnr_k)
-  DevBuf<unsigned> srnr_list, srnr_count;
+  DevBuf<unsigned> srnr_list;
   DevBuf<int> srnr_row_of, srnr_row_site;
   DevBuf<int32_t> knn2;
   // cells of the cell -> tet form
@@ -420,7 +423,7 @@ int vd_ctx_create(vd_ctx** out, int device, const vd_config* cfg) {
   }
   for (auto& row : ctx->ev)
     for (auto& e : row) (void)hipEventCreate(&e);
-  if (ensure_offsets(ctx) != VD_OK || ctx->hist.ensure(vd::kHistWords) != hipSuccess) {
+  if (ensure_offsets(ctx) != VD_OK || ctx->hist.ensure(vd_ctx::kCounterWords / 2) != hipSuccess) {
     fprintf(stderr, "vd_ctx_create: %s\n", ctx->err.c_str());
     vd_ctx_destroy(ctx);
     return VD_ERR_HIP;
@@ -445,10 +448,10 @@ void vd_ctx_destroy(vd_ctx* ctx) {
   ctx->p_count.release(); ctx->p_start.release(); ctx->p_cursor.release(); ctx->p_ids.release(); ctx->p_surv.release();
   ctx->acc_f32.release(); ctx->acc_fix.release(); ctx->moments.release();
   ctx->pair_status.release(); ctx->pair_vals.release(); ctx->hist.release();
-  ctx->retry_list.release(); ctx->retry_count.release(); ctx->retry_list2.release(); ctx->retry_count2.release(); ctx->site_counter.release();
-  ctx->srnr_list.release(); ctx->srnr_count.release(); ctx->srnr_row_of.release(); ctx->srnr_row_site.release();
+  ctx->retry_list.release(); ctx->retry_list2.release();
+  ctx->srnr_list.release(); ctx->srnr_row_of.release(); ctx->srnr_row_site.release();
   ctx->knn2.release();
-  ctx->rec_meta.release(); ctx->rec_tris.release(); ctx->rec_count.release();
+  ctx->rec_meta.release(); ctx->rec_tris.release();
   ctx->c_status.release(); ctx->c_nv.release(); ctx->c_nt.release(); ctx->c_r2.release();
   ctx->c_planes.release(); ctx->c_tris.release(); ctx->c_redo.release();
   for (auto& row : ctx->ev)
@@ -743,14 +746,21 @@ int vd_clip_step(vd_ctx* ctx) {
                      "mesh volume x largest |coordinate| = %.3g exceeds %.3g, the range of the exact FP64 "
                      "fixed-point sums: map the mesh into the [0,1000]^3 frame or use VD_ACCUM_F32",
                      ctx->fixed_load, vdi::kFixedPointMaxLoad);
+  const bool by_site = c.form == VD_FORM_SITE_MAJOR || c.form == VD_FORM_CELLS;
+  vd::ClearList clear;
   if (c.accum == VD_ACCUM_F32) {
     VD_HIP(ctx->acc_f32.ensure(4 * (size_t)n), "alloc acc");
-    VD_HIP(vd::fill_u32(ctx->acc_f32.p, 4LL * n, 0u, ctx->stream), "clear acc");
+    clear.add(ctx->acc_f32.p, 4LL * n);
   } else {
     VD_HIP(ctx->acc_fix.ensure(4 * (size_t)n), "alloc acc");
-    VD_HIP(vd::fill_u32(ctx->acc_fix.p, 8LL * n, 0u, ctx->stream), "clear acc");
+    clear.add(ctx->acc_fix.p, 8LL * n);
   }
-  VD_HIP(vd::fill_u32(ctx->hist.p, 2 * vd::kHistWords, 0u, ctx->stream), "clear hist");
+  clear.add(ctx->hist.p, vd_ctx::kCounterWords);
+  if (by_site) {
+    VD_HIP(ctx->p_count.ensure(n), "alloc pairs");
+    clear.add(ctx->p_count.p, n);
+  }
+  VD_HIP(vd::clear_all(clear, ctx->stream), "clear");
   if (c.record_pairs) {
     VD_HIP(ctx->pair_status.ensure(std::max(n_pairs, 1LL)), "alloc pair status");
     VD_HIP(ctx->pair_vals.ensure(4 * std::max(n_pairs, 1LL)), "alloc pair vals");
@@ -776,13 +786,11 @@ int vd_clip_step(vd_ctx* ctx) {
   a.status_hist = ctx->hist.p;
   a.filter = c.filter;
   int blocks = 0;
-  if (c.form == VD_FORM_SITE_MAJOR || c.form == VD_FORM_CELLS) {
-    VD_HIP(ctx->p_count.ensure(n), "alloc pairs");
+  if (by_site) {
     VD_HIP(ctx->p_start.ensure((size_t)n + 1), "alloc pairs");
     VD_HIP(ctx->p_cursor.ensure(n), "alloc pairs");
     VD_HIP(ctx->p_ids.ensure(std::max(n_pairs, 1LL)), "alloc pairs");
     VD_HIP(ctx->p_scan_tmp.ensure(vd::scan_tmp_ints(n)), "alloc pairs");
-    VD_HIP(vd::fill_u32(ctx->p_count.p, n, 0u, ctx->stream), "clear pairs");
     VD_HIP(vd::pairs_by_site(ctx->tet_knn.p, n_pairs, n, ctx->p_count.p, ctx->p_start.p, ctx->p_cursor.p, ctx->p_ids.p,
                              ctx->p_scan_tmp.p, ctx->stream),
            "pairs by site");
@@ -815,9 +823,7 @@ int vd_clip_step(vd_ctx* ctx) {
       return VD_OK;
     }
     blocks = c.clip_blocks;
-    VD_HIP(ctx->site_counter.ensure(1), "alloc site counter");
-    VD_HIP(vd::fill_u32(ctx->site_counter.p, 1, 0u, ctx->stream), "clear site counter");
-    a.site_counter = ctx->site_counter.p;
+    a.site_counter = ctx->counter(vd_ctx::kSiteCounter);
     const int fast_tcap = vdi::site_tcap_of(c);
     a.site_depth = site_depth_of(c, ctx->K);
     if (ctx->fresh_sites && c.site_depth == 0) a.site_depth = std::min(kFreshSiteDepth, ctx->K);
@@ -829,10 +835,8 @@ int vd_clip_step(vd_ctx* ctx) {
     if (fast_tcap < c.tcap || std::min(a.site_depth, site_depth_of(c, ctx->K)) < ctx->K ||
         c.moments == VD_MOMENTS_ROBUST) {
       VD_HIP(ctx->retry_list.ensure(std::max(n_pairs, 1LL)), "alloc retry list");
-      VD_HIP(ctx->retry_count.ensure(1), "alloc retry list");
-      VD_HIP(vd::fill_u32(ctx->retry_count.p, 1, 0u, ctx->stream), "clear retry count");
       a.retry_list = ctx->retry_list.p;
-      a.retry_count = ctx->retry_count.p;
+      a.retry_count = ctx->counter(vd_ctx::kRetryCount);
     }
     a.tcap = fast_tcap;
     a.tcap_full = c.tcap;
@@ -851,11 +855,9 @@ int vd_clip_step(vd_ctx* ctx) {
       const unsigned cap = (unsigned)std::max(1LL, std::min({want, n_pairs, (long long)UINT32_MAX}));
       VD_HIP(ctx->rec_meta.ensure(cap), "alloc records");
       VD_HIP(ctx->rec_tris.ensure((size_t)cap * vd::rec_stride(fast_tcap)), "alloc records");
-      VD_HIP(ctx->rec_count.ensure(1), "alloc records");
-      VD_HIP(vd::fill_u32(ctx->rec_count.p, 1, 0u, ctx->stream), "clear record count");
       a.rec_meta = ctx->rec_meta.p;
       a.rec_tris = ctx->rec_tris.p;
-      a.rec_count = ctx->rec_count.p;
+      a.rec_count = ctx->counter(vd_ctx::kRecCount);
       a.rec_cap = cap;
     }
   } else {
@@ -872,10 +874,8 @@ int vd_clip_step(vd_ctx* ctx) {
   }
   if (K2 > 0) {
     VD_HIP(ctx->srnr_list.ensure(std::max(n_pairs, 1LL)), "alloc srnr list");
-    VD_HIP(ctx->srnr_count.ensure(2), "alloc srnr list");
-    VD_HIP(vd::fill_u32(ctx->srnr_count.p, 2, 0u, ctx->stream), "clear srnr list");
     a.srnr_list = ctx->srnr_list.p;
-    a.srnr_count = ctx->srnr_count.p;
+    a.srnr_count = ctx->counter(vd_ctx::kSrnrCount);
   }
   // The site-major form's re-clip of its overflow pairs depends on the
   // clipping launch only: it runs on the second stream beside the volume pass
@@ -911,17 +911,15 @@ int vd_clip_step(vd_ctx* ctx) {
       r.pcap_full = c.pcap;
       if (mid < c.tcap || pmid < c.pcap) {
         VD_HIP(ctx->retry_list2.ensure(std::max(n_pairs, 1LL)), "alloc retry list");
-        VD_HIP(ctx->retry_count2.ensure(1), "alloc retry list");
-        VD_HIP(vd::fill_u32(ctx->retry_count2.p, 1, 0u, rs), "clear retry count");
         r.retry_list = ctx->retry_list2.p;
-        r.retry_count = ctx->retry_count2.p;
+        r.retry_count = ctx->counter(vd_ctx::kRetryCount2);
       }
       VD_HIP(vd::clip_launch(r, vd::kFormTetCached, c.moments, c.accum, 768, rs), "clip retry");
       if (mid < c.tcap || pmid < c.pcap) {
         vd::ClipArgs r3 = a;
         r3.tcap = c.tcap;
         r3.pair_list = ctx->retry_list2.p;
-        r3.pair_list_count = ctx->retry_count2.p;
+        r3.pair_list_count = ctx->counter(vd_ctx::kRetryCount2);
         r3.retry_list = nullptr;
         r3.retry_count = nullptr;
         VD_HIP(vd::clip_launch(r3, VD_FORM_TET_MAJOR, c.moments, c.accum, 256, rs), "clip retry");
@@ -940,8 +938,8 @@ int vd_clip_step(vd_ctx* ctx) {
     VD_HIP(ctx->srnr_row_site.ensure(n), "alloc srnr rows");
     VD_HIP(ctx->knn2.ensure((size_t)n * K2), "alloc srnr rows");
     VD_HIP(vd::fill_u32(ctx->srnr_row_of.p, n, 0xffffffffu, ctx->stream), "clear srnr rows");
-    unsigned* n_rows = ctx->srnr_count.p + 1;
-    VD_HIP(vd::srnr_rows(ctx->srnr_list.p, ctx->srnr_count.p, n_pairs, ctx->tet_knn.p, n, ctx->srnr_row_of.p,
+    unsigned* n_rows = ctx->counter(vd_ctx::kSrnrCount) + 1;
+    VD_HIP(vd::srnr_rows(ctx->srnr_list.p, ctx->counter(vd_ctx::kSrnrCount), n_pairs, ctx->tet_knn.p, n, ctx->srnr_row_of.p,
                          ctx->srnr_row_site.p, n_rows, ctx->stream),
            "srnr rows");
     VD_HIP(vd::knn_query_ids(grid_bufs(ctx), ctx->offsets.p, ctx->n_offsets, K2, ctx->sites.p, ctx->srnr_row_site.p,
@@ -950,7 +948,7 @@ int vd_clip_step(vd_ctx* ctx) {
     vd::ClipArgs r = a;
     r.tcap = c.tcap;
     r.pair_list = ctx->srnr_list.p;
-    r.pair_list_count = ctx->srnr_count.p;
+    r.pair_list_count = ctx->counter(vd_ctx::kSrnrCount);
     r.retry_list = nullptr;
     r.retry_count = nullptr;
     r.srnr_list = nullptr;

@@ -1062,6 +1062,21 @@ hipError_t fill_u32(void* p, long long n, uint32_t v, hipStream_t st) {
   return hipGetLastError();
 }
 
+__global__ void k_clear(ClearList l) {
+  for (int i = 0; i < l.n; ++i)
+    for (long long j = (long long)blockIdx.x * blockDim.x + threadIdx.x; j < l.words[i];
+         j += (long long)gridDim.x * blockDim.x)
+      l.p[i][j] = 0u;
+}
+
+hipError_t clear_all(const ClearList& l, hipStream_t st) {
+  long long most = 0;
+  for (int i = 0; i < l.n; ++i) most = std::max(most, l.words[i]);
+  if (most <= 0) return hipSuccess;
+  hipLaunchKernelGGL(k_clear, dim3((unsigned)std::min<long long>((most + 255) / 256, 4096)), dim3(256), 0, st, l);
+  return hipGetLastError();
+}
+
 // Exclusive scan, three passes: per-block scans of kScanTile items, a scan of
 // the block totals, then the block offsets added back.  Also clears `cursor`.
 constexpr int kScanItems = 8;
