@@ -1229,9 +1229,10 @@ __global__ __launch_bounds__(64) void k_clip_plain(ClipArgs a) {
 //
 // Pairs grouped by seed: site s owns pair_ids[pair_start[s] .. pair_start[s+1]),
 // or the first pair_count[s] of them when the emptiness test (k_cull_site)
-// has run.  A wavefront takes sites one at a time from a global counter.  For
-// each site it builds the bisector table once (shared by the wave) and queues
-// the site's pairs in an LDS ring.  Every lane clips its own pair a few
+// has run.  A wavefront takes work units (a run of one site's pairs,
+// site_units) one at a time from a global counter.  For each site it builds
+// the bisector table (shared by the wave) and queues the unit's pairs in an
+// LDS ring.  Every lane clips its own pair a few
 // bisectors per loop trip and takes the next queued pair as soon as it is
 // done, so lanes do not wait for the slowest pair of a group.  Two table slots let lanes start on the next site
 // while others finish the previous one.  Tet corners come from a per-tet
@@ -1296,11 +1297,13 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
 
   // wave-uniform scheduling state
   int site0 = -1, site1 = -1;         // site of each table slot
-  int feed_slot = 1;                  // slot of the site being fed into the queue
-  unsigned cursor = 0, feed_end = 0;  // its pairs not yet through the emptiness test
+  int feed_slot = 1;                  // slot of the unit being fed into the queue
+  unsigned cursor = 0, feed_end = 0;  // its pairs not yet queued
   unsigned qhead = 0, qtail = 0;      // queue ring positions
   unsigned qsplit = 0;                // entries before qsplit belong to the other slot
-  bool no_more_sites = false;
+  const unsigned n_units = *a.unit_count;
+  bool no_more_units = false;
+  uint4 next_unit = make_uint4(0u, 0u, 0u, 0u);  // taken, not yet fed (z: its pairs)
 
   // lane state
   int lst = kIdle;
@@ -1311,59 +1314,64 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
   unsigned rec_next0 = 0, rec_end0 = 0, rec_next1 = 0, rec_end1 = 0;  // wave-uniform
 
   for (;;) {
-    // (1) refill the queue up to 64 entries
-    while (qtail - qhead < 64) {
+    // (1) refill the queue while it holds fewer entries than lanes are idle (a
+    // wave that took pairs ahead would hold them while other waves run dry)
+    const unsigned long long idle = __ballot(lst == kIdle);
+    const unsigned n_idle = (unsigned)__popcll(idle);
+    while (qtail - qhead < n_idle) {
       if (cursor < feed_end) {
         __syncthreads();  // queue entries read by the previous trip
         const unsigned i = cursor + lane;
         const bool live = i < feed_end;
         const unsigned pair = live ? a.pair_ids[i] : 0u;
-        const unsigned long long mask = __ballot(live);
-        const int below = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-        if (live) queue[(qtail + (unsigned)below) % kQueue] = pair;
-        qtail += (unsigned)__popcll(mask);
-        cursor += 64;
+        if (live) queue[(qtail + lane) % kQueue] = pair;
+        const unsigned n = min(64u, feed_end - cursor);
+        qtail += n;
+        cursor += n;
         continue;
       }
-      if (no_more_sites) break;
-      // the other slot is free once no lane and no queued entry refers to it
-      const int other = feed_slot ^ 1;
-      if (__ballot(lst != kIdle && pslot == other) != 0 || qhead < qsplit) break;
-      int s = 0;
-      if (lane == 0) s = (int)atomicAdd(a.site_counter, 1u);
-      s = __builtin_amdgcn_readfirstlane(s);
-      if (s >= a.n_sites) {
-        no_more_sites = true;
-        break;
-      }
-      if (a.site_order) s = a.site_order[s];
-      const unsigned pb = a.pair_start[s], pe = a.pair_count ? pb + a.pair_count[s] : a.pair_start[s + 1];
-      if (pb == pe) continue;
-      const P4 sp = site_at(a, s);
-      const int32_t* nbr = a.site_knn + (size_t)s * a.K;
-      __syncthreads();  // the slot's last readers are done
-      float4* eb = bis + other * K4;
-      for (int v = lane; v < K; v += 64) {
-        const int z = nbr[v];
-        if ((unsigned)z >= (unsigned)a.n_sites) {  // clipping stops at such a neighbour
-          const float nan = __int_as_float(0x7fc00000);
-          eb[v] = make_float4(nan, nan, nan, nan);
-          continue;
+      if (next_unit.z == 0u) {
+        if (no_more_units) break;
+        unsigned u = 0;
+        if (lane == 0) u = atomicAdd(a.site_counter, 1u);
+        u = (unsigned)__builtin_amdgcn_readfirstlane((int)u);
+        if (u >= n_units) {
+          no_more_units = true;
+          break;
         }
-        const P4 eq = bisector(sp, site_at(a, z));
-        eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w);
+        next_unit = a.units[u];
       }
-      __syncthreads();
-      if (other) site1 = s; else site0 = s;
-      feed_slot = other;
-      cursor = pb;
-      feed_end = pe;
-      qsplit = qtail;
+      const int s = (int)next_unit.x;
+      if (s != (feed_slot ? site1 : site0)) {
+        // the other slot is free once no lane and no queued entry refers to it
+        const int other = feed_slot ^ 1;
+        if (__ballot(lst != kIdle && pslot == other) != 0 || qhead < qsplit) break;
+        const P4 sp = site_at(a, s);
+        const int32_t* nbr = a.site_knn + (size_t)s * a.K;
+        __syncthreads();  // the slot's last readers are done
+        float4* eb = bis + other * K4;
+        for (int v = lane; v < K; v += 64) {
+          const int z = nbr[v];
+          if ((unsigned)z >= (unsigned)a.n_sites) {  // clipping stops at such a neighbour
+            const float nan = __int_as_float(0x7fc00000);
+            eb[v] = make_float4(nan, nan, nan, nan);
+            continue;
+          }
+          const P4 eq = bisector(sp, site_at(a, z));
+          eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w);
+        }
+        __syncthreads();
+        if (other) site1 = s; else site0 = s;
+        feed_slot = other;
+        qsplit = qtail;
+      }
+      cursor = next_unit.y;
+      feed_end = next_unit.y + next_unit.z;
+      next_unit.z = 0u;
     }
     __syncthreads();
 
     // (2) idle lanes take queued pairs in queue order
-    const unsigned long long idle = __ballot(lst == kIdle);
     const unsigned avail = qtail - qhead;
     const unsigned rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0));
     if (lst == kIdle && rank < avail) {
@@ -1377,10 +1385,10 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
       c.ps.bis = bis + pslot * K4;
       c.init_tet_prep(site_at(a, pslot ? site1 : site0), a.tet_prep + kTetPrepWords * (size_t)ptet);
     }
-    qhead += min((unsigned)__popcll(idle), avail);
+    qhead += min(n_idle, avail);
     const int n_clip = __popcll(__ballot(lst == kClipping));
     if (n_clip == 0) {
-      if (no_more_sites && cursor >= feed_end && qhead == qtail) break;
+      if (no_more_units && next_unit.z == 0u && cursor >= feed_end && qhead == qtail) break;
       continue;
     }
     // Result of a finished pair: retry entry, or accumulation and records.
@@ -1753,6 +1761,46 @@ __global__ __launch_bounds__(64) void k_cull_site(ClipArgs a, int depth, unsigne
     if (lane == 0) pair_count[s] = w - pb;
   }
   if (lane == 0 && a.status_hist && n_culled) add_status(a, kNoIntersection, n_culled);
+}
+
+// The work units of the site-major clipping (site_units): with whole sites as
+// the unit, a wave that got a site of several thousand pairs (a sparse region's
+// large cell) ran on alone, and with fewer sites than the GPU holds waves the
+// others had none.  The clipping at 820k torus tets / 200,000 clustered sites
+// took 19.6 ms and 9.9 ms (iterations 1 and 2), now 9.0 and 6.6; at 48,000 tets /
+// 2,000 sites 521 us, now 329.  8 us at 100,000 sites.
+constexpr int kUnitThreads = 256;
+__global__ __launch_bounds__(kUnitThreads) void k_site_units(ClipArgs a, unsigned unit_pairs, uint4* units,
+                                                             unsigned* unit_count) {
+  __shared__ unsigned wsum[kUnitThreads / 64];
+  __shared__ unsigned base;
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int si = blockIdx.x * kUnitThreads + tid;
+  int s = 0;
+  unsigned pb = 0, n = 0;
+  if (si < a.n_sites) {
+    s = a.site_order ? a.site_order[si] : si;
+    pb = a.pair_start[s];
+    n = a.pair_count ? a.pair_count[s] : a.pair_start[s + 1] - pb;
+  }
+  const unsigned mine = (n + unit_pairs - 1u) / unit_pairs;
+  unsigned incl = mine;
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const unsigned v = __shfl_up(incl, d);
+    if (lane >= d) incl += v;
+  }
+  if (lane == 63) wsum[wv] = incl;
+  __syncthreads();
+  unsigned before = incl - mine, total = 0;
+  for (int w = 0; w < kUnitThreads / 64; ++w) {
+    if (w < wv) before += wsum[w];
+    total += wsum[w];
+  }
+  if (tid == 0 && total) base = atomicAdd(unit_count, total);
+  __syncthreads();
+  for (unsigned u = 0; u < mine; ++u)
+    units[base + before + u] = make_uint4((unsigned)s, pb + u * unit_pairs, min(unit_pairs, n - u * unit_pairs), 0u);
 }
 
 // Volume pass of the site-major form: one lane per record.  The planes are
@@ -2501,7 +2549,6 @@ static hipError_t launch_site(Kern k, int n_blocks, size_t lds, hipStream_t st, 
     if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
     n_blocks = std::max(1, per_cu * cus);
   }
-  n_blocks = std::max(1, std::min(n_blocks, a.n_sites));
   hipLaunchKernelGGL(k, dim3((unsigned)n_blocks), dim3(64), lds, st, a);
   return hipGetLastError();
 }
@@ -2528,7 +2575,7 @@ hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, i
     if (moments == 1 && acc_mode == 0) return launch_lds(k_clip_plain<1, 0, 1>, grid, block, lds, st, a);
     return launch_lds(k_clip_plain<1, 1, 1>, grid, block, lds, st, a);
   }
-  if (!a.site_counter) return hipErrorInvalidValue;
+  if (!a.site_counter || !a.units || !a.unit_count) return hipErrorInvalidValue;
   if (a.rec_meta && (!a.rec_tris || !a.rec_count)) return hipErrorInvalidValue;
   // the robust moments are never computed in the site-major kernel: the
   // polytopes it cannot hand to the volume pass go to the retry list
@@ -2585,6 +2632,14 @@ hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* pair_coun
   const unsigned blocks =
       (unsigned)(kXcds * std::max(1, std::min((a.n_sites + kXcds - 1) / kXcds, VD_CULL_BLOCKS / kXcds)));
   hipLaunchKernelGGL(k_cull_site, dim3(blocks), dim3(64), 32 * (size_t)depth, st, a, depth, pair_ids, pair_count);
+  return hipGetLastError();
+}
+
+hipError_t site_units(const ClipArgs& a, int unit_pairs, uint4* units, unsigned* unit_count, hipStream_t st) {
+  if (a.n_sites <= 0) return hipSuccess;
+  if (unit_pairs < 1) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_site_units, dim3((unsigned)((a.n_sites + kUnitThreads - 1) / kUnitThreads)), dim3(kUnitThreads),
+                     0, st, a, (unsigned)unit_pairs, units, unit_count);
   return hipGetLastError();
 }
 

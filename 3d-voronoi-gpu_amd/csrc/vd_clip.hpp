@@ -38,8 +38,10 @@ struct ClipArgs {
   int cull_depth;            // cull_sites and the cell form: bisectors tried by the emptiness
                              // test (0 = off)
   int filter;                // arithmetic filter of the conflict test (0 off, 1 reference, 2 FP64 re-check)
-  unsigned* site_counter;    // site-major form: next site to take, zero before the launch
-  const int* site_order;     // site-major form and cull_sites, optional: the order in which sites are
+  unsigned* site_counter;    // site-major form: next unit to take, zero before the launch
+  const uint4* units;        // site-major form: the work units (site_units)
+  const unsigned* unit_count;  // with units: their number
+  const int* site_order;     // cull_sites and site_units, optional: the order in which sites are
                              // taken (a permutation; neighbouring sites next to each other share
                              // tets, which then stay in cache)
   int site_depth;            // site-major form: bisectors per site table (0 = K); a pair
@@ -142,6 +144,15 @@ inline int exact_cull_depth(int depth, int pcap, int tcap) {
 // range and their number written to pair_count[s]; a culled pair counts as
 // no_intersection (a.status_hist, a.pair_status, a.pair_vals).
 hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* pair_count, hipStream_t st);
+// The work units of the site-major clipping: every site's pairs (the first
+// pair_count[s] of its range when given, else all) cut into runs of at most
+// unit_pairs, each (site, first pair position, number of pairs, 0), in the
+// order of a.site_order within every 256 sites.  *unit_count must be zero;
+// units holds max_site_units(...) entries.
+inline long long max_site_units(long long n_pairs, int n_sites, int unit_pairs) {
+  return n_sites + n_pairs / unit_pairs;
+}
+hipError_t site_units(const ClipArgs& a, int unit_pairs, uint4* units, unsigned* unit_count, hipStream_t st);
 // Per tet of the corner records tet_xyz[0..3n): its face planes (ids 0..3) and
 // the FP32 vertices of its four start triangles, 7 float4 per tet
 // (kTetPrepWords), so that a pair's start loads them instead of computing

@@ -165,6 +165,7 @@ struct vd_ctx {
   // site-major pairs
   DevBuf<int> p_count, p_cursor;
   DevBuf<unsigned> p_start, p_ids;
+  DevBuf<uint4> units;      // work units of the clipping
   DevBuf<unsigned> p_surv;  // survivors of the emptiness test per site
   // accumulators
   DevBuf<float> acc_f32;
@@ -175,7 +176,7 @@ struct vd_ctx {
   // the status counters (vd::kHistWords) and then the step's other counters,
   // each in a cache line of its own, cleared together
   DevBuf<unsigned long long> hist;
-  enum Counter { kSiteCounter, kRetryCount, kRetryCount2, kRecCount, kSrnrCount, kCounters };
+  enum Counter { kUnitCounter, kUnitCount, kRetryCount, kRetryCount2, kRecCount, kSrnrCount, kCounters };
   static constexpr int kCounterStride = 32;
   static constexpr int kCounterWords = 2 * vd::kHistWords + kCounters * kCounterStride;
   unsigned* counter(Counter c) { return (unsigned*)hist.p + 2 * vd::kHistWords + c * kCounterStride; }
@@ -445,7 +446,7 @@ void vd_ctx_destroy(vd_ctx* ctx) {
   ctx->g_cell_of.release(); ctx->g_sorted_ids.release(); ctx->g_sorted_pts.release();
   ctx->g_scan_tmp.release(); ctx->p_scan_tmp.release();
   ctx->site_knn.release(); ctx->tet_knn.release();
-  ctx->p_count.release(); ctx->p_start.release(); ctx->p_cursor.release(); ctx->p_ids.release(); ctx->p_surv.release();
+  ctx->p_count.release(); ctx->p_start.release(); ctx->p_cursor.release(); ctx->p_ids.release(); ctx->p_surv.release(); ctx->units.release();
   ctx->acc_f32.release(); ctx->acc_fix.release(); ctx->moments.release();
   ctx->pair_status.release(); ctx->pair_vals.release(); ctx->hist.release();
   ctx->retry_list.release(); ctx->retry_list2.release();
@@ -823,7 +824,7 @@ int vd_clip_step(vd_ctx* ctx) {
       return VD_OK;
     }
     blocks = c.clip_blocks;
-    a.site_counter = ctx->counter(vd_ctx::kSiteCounter);
+    a.site_counter = ctx->counter(vd_ctx::kUnitCounter);
     const int fast_tcap = vdi::site_tcap_of(c);
     a.site_depth = site_depth_of(c, ctx->K);
     if (ctx->fresh_sites && c.site_depth == 0) a.site_depth = std::min(kFreshSiteDepth, ctx->K);
@@ -849,6 +850,17 @@ int vd_clip_step(vd_ctx* ctx) {
       a.pair_count = ctx->p_surv.p;
       a.cull_depth = 0;
     }
+    // Pairs per work unit of the clipping: a wave serves two sites at a time, so
+    // units much below 64 pairs leave its lanes idle, and units that split most
+    // sites build their tables twice.  ms at 1M tets / 100,000 sites (10
+    // iterations), 820k torus tets (2), 48,000 tets / 2,000 sites (1): 32 pairs
+    // 93.9, 47.7, 1.12; 64 79.3, 44.9, 1.04; 128 75.3, 44.2, 1.06; 256 75.2,
+    // 44.5, 1.16; 1,024 75.3, 45.7, 1.24.
+    const int unit = n < 8192 ? 64 : 128;
+    VD_HIP(ctx->units.ensure((size_t)vd::max_site_units(n_pairs, n, unit)), "alloc units");
+    VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
+    a.units = ctx->units.p;
+    a.unit_count = ctx->counter(vd_ctx::kUnitCount);
     if (c.site_records >= 0) {
       // automatic: one pair in ten, plus the slots the waves reserve ahead
       const long long want = c.site_records > 0 ? c.site_records : n_pairs / 10 + 262144;
@@ -889,9 +901,9 @@ int vd_clip_step(vd_ctx* ctx) {
     VD_HIP(hipEventRecord(ctx->fork_ev, ctx->stream), "event");
     VD_HIP(hipStreamWaitEvent(ctx->side, ctx->fork_ev, 0), "stream wait");
     rs = ctx->side;
-    VD_HIP(vd::site_volume_pass(a, c.moments, c.accum, ctx->stream), "volume pass");
+  } else {
+    VD_HIP(record_phase(ctx, (5)), "event");
   }
-  VD_HIP(record_phase(ctx, (5)), "event");
   if (a.retry_list) {
     // pairs that overflowed the site-major launch's vertex cap or needed more
     // bisectors than its tables hold: re-clipped by the tet-major kernel with
@@ -931,6 +943,11 @@ int vd_clip_step(vd_ctx* ctx) {
   }
   if (beside) {
     VD_HIP(hipEventRecord(ctx->join_ev, ctx->side), "event");
+    // The volume pass is enqueued after the re-clip: the re-clip's workgroups
+    // need 51 KB of LDS each, and behind the volume pass's thousands of small
+    // ones they get in only as those run out.
+    VD_HIP(vd::site_volume_pass(a, c.moments, c.accum, ctx->stream), "volume pass");
+    VD_HIP(record_phase(ctx, (5)), "event");
     VD_HIP(hipStreamWaitEvent(ctx->stream, ctx->join_ev, 0), "stream wait");
   }
   if (K2 > 0) {
