@@ -61,6 +61,15 @@ int site_depth_of(const vd_config& c, int K) { return std::min(c.site_depth > 0 
 // re-clip from scratch cost more than the deeper tables' lost occupancy (one
 // wave per CU fewer at the same vertex cap).
 constexpr int kFreshSiteDepth = 64;
+// Below this many nonempty (tet, cell) pieces (vdi::pieces_estimate) the
+// clipping's waves do not fill the GPU several times over, and what counts is
+// the longest chain of launches: the site-major launch then runs at caps that
+// leave nearly nothing to the re-clip (32 vertices, tables of all neighbours
+// up to 96; 5 waves per CU at 90 instead of 9).  Clipping ms per iteration,
+// wide against the automatic caps: 10,368 tets 0.32 / 0.43, 24,576 0.42 / 0.58,
+// 48,000 0.60 / 0.69, 82,944 (386k pieces) 0.80 / 0.77, 146,334 1.25 / 1.14.
+constexpr double kWidePieces = 256e3;
+constexpr int kWideDepth = 96, kWideTcap = 32;
 // kNN steps after the caller sets sites that do without the previous rows'
 // bounds (see vd_knn_step)
 constexpr int kHintAfter = 2;
@@ -99,6 +108,12 @@ double fixed_point_load(const float* verts_xyz, int v0, int nv, const int32_t* t
            6.0;
   }
   return vol * m;
+}
+
+double pieces_estimate(double n_tets, double n_sites) {
+  if (!(n_tets > 0.0)) return 0.0;
+  const double e = 1.0 + 1.44 * std::cbrt(std::max(n_sites, 0.0) / n_tets);
+  return n_tets * e * e * e;
 }
 
 int site_tcap_of(const vd_config& c) {
@@ -825,9 +840,14 @@ int vd_clip_step(vd_ctx* ctx) {
     }
     blocks = c.clip_blocks;
     a.site_counter = ctx->counter(vd_ctx::kUnitCounter);
-    const int fast_tcap = vdi::site_tcap_of(c);
+    int fast_tcap = vdi::site_tcap_of(c);
     a.site_depth = site_depth_of(c, ctx->K);
-    if (ctx->fresh_sites && c.site_depth == 0) a.site_depth = std::min(kFreshSiteDepth, ctx->K);
+    if (c.site_tcap == 0 && c.site_depth == 0 && vdi::pieces_estimate(ctx->n_tets, n) <= kWidePieces) {
+      fast_tcap = std::min(c.tcap, kWideTcap);
+      a.site_depth = std::min(kWideDepth, ctx->K);
+    } else if (ctx->fresh_sites && c.site_depth == 0) {
+      a.site_depth = std::min(kFreshSiteDepth, ctx->K);
+    }
     ctx->fresh_sites = false;
     // (the robust moments also need it: the site-major kernel retries the
     // polytopes it cannot hand to the volume pass; and it is allocated alike

@@ -42,6 +42,10 @@ int assemble(vd_ctx* ctx, const JobDev* jobs, int n);
 int scatter_sites(vd_ctx* ctx, const JobDev* jobs, const int* idx, int n_idx);
 hipStream_t stream(vd_ctx* ctx);
 void set_error(vd_ctx* ctx, const char* msg);
+// Nonempty intersections of n_tets tets with the cells of n_sites sites, about:
+// 4.65 per tet at a tenth as many sites (counted: 4.60 at 998,250 tets, 4.65
+// at 146,334), growing as the cells shrink against the tets.
+double pieces_estimate(double n_tets, double n_sites);
 // Vertex cap of the site-major launch under configuration c (its site_tcap,
 // or the automatic choice).
 int site_tcap_of(const vd_config& c);

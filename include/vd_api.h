@@ -73,7 +73,8 @@ typedef struct vd_config {
                          exceed it are recomputed at tcap, so results do not depend
                          on it; 0 = automatic: the largest (at most 32) whose LDS at
                          the configured table depth lets 9 waves share a CU, 17 at
-                         site_depth 40 */
+                         site_depth 40; with site_depth 0 too, 32 on a small problem (about
+                         55,000 tets with a tenth as many sites, all instances together) */
   int cull_depth;     /* site-major form: a pair whose tet lies entirely beyond one of the
                          seed's first cull_depth bisectors (by more than the FP32 rounding
                          bound plus 0.01) has an empty intersection and is not clipped
@@ -101,7 +102,8 @@ typedef struct vd_config {
                          needs more is recomputed from scratch at site_k by the retry pass,
                          so results do not depend on it; 0 = automatic (40, and 64 for the
                          first clipping after vd_set_sites or vd_set_batch: sites not yet
-                         moved by an update need deeper tables) */
+                         moved by an update need deeper tables; with site_tcap 0 too, 96 on
+                         a small problem) */
   int knn_waves;      /* wavefronts per workgroup of the kNN queries: 2, 4 or 8; 0 = automatic
                          (4); results do not depend on it */
   int cells_pcap;     /* cell form: plane cap of kernel B's first launch (8..pcap); cells that

@@ -26,3 +26,22 @@ def test_units_bit_exact(vdn, O, n, ns, tk, cull):
             np.testing.assert_array_equal(vals, r["pair_vals"])
             np.testing.assert_array_equal(mom, r["site_vals"])
             assert [hist[k] for k in vdn.STATUS_NAMES] == np.bincount(r["pair_status"], minlength=7).tolist()
+
+
+@pytest.mark.parametrize("n,ns", [(3, 40), (21, 5000), (21, 5800)])
+def test_small_problem_caps(vdn, O, n, ns):
+    """The automatic caps below and above the small-problem limit (256,000
+    estimated pieces: 55,566 tets with 5,000 and 5,800 sites lie on its two
+    sides) and the same caps given by hand: one result, the oracle's."""
+    verts, tets, sites = problem("cube", n, ns)
+    tk = min(64, ns)
+    sk, tkn = oracle_knn("cube", n, ns, 90, tk)
+    r = O.clip_tets(sites, sk, verts, tets, tkn, geom="f32", pair_acc="f64", site_mode=O.SITE_FIXED, moments="robust",
+                    want_pairs=False)
+    for cfg in ({}, {"site_tcap": 32, "site_depth": 90}, {"site_tcap": 17, "site_depth": 40}):
+        with vdn.Engine(tet_k=tk, accum="f64", moments="robust", **cfg) as e:
+            e.set_mesh(verts, tets)
+            e.set_sites(sites)
+            e.knn_step()
+            e.clip_step()
+            np.testing.assert_array_equal(e.moments(), r["site_vals"])
