@@ -12,6 +12,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -116,6 +117,11 @@ double pieces_estimate(double n_tets, double n_sites) {
   return n_tets * e * e * e;
 }
 
+double records_per_tet(double n_tets, double n_sites, int TK) {
+  if (!(n_tets > 0.0)) return 0.0;
+  return std::min((double)TK, std::max(TK / 10.0, 1.3 * pieces_estimate(n_tets, n_sites) / n_tets));
+}
+
 int site_tcap_of(const vd_config& c) {
   if (c.site_tcap > 0) return std::min(c.site_tcap, c.tcap);
   const int depth = std::max(site_depth_of(c, c.site_k), 1);
@@ -200,6 +206,7 @@ struct vd_ctx {
   // site-major form: records of finished polytopes for the volume pass
   DevBuf<uint4> rec_meta;
   DevBuf<uint32_t> rec_tris;
+  long long more_records = LLONG_MAX;  // records beyond a tenth of the pairs, at most (vdi::limit_records)
   // pairs retried with deeper neighbour lists (srnr_k)
   DevBuf<unsigned> srnr_list;
   DevBuf<int> srnr_row_of, srnr_row_site;
@@ -882,8 +889,12 @@ int vd_clip_step(vd_ctx* ctx) {
     a.units = ctx->units.p;
     a.unit_count = ctx->counter(vd_ctx::kUnitCount);
     if (c.site_records >= 0) {
-      // automatic: one pair in ten, plus the slots the waves reserve ahead
-      const long long want = c.site_records > 0 ? c.site_records : n_pairs / 10 + 262144;
+      // automatic: the estimate, plus the slots the waves reserve ahead
+      const long long more =
+          (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
+      const long long want = c.site_records > 0
+                                 ? c.site_records
+                                 : n_pairs / 10 + std::max(0LL, std::min(more, ctx->more_records)) + 262144;
       const unsigned cap = (unsigned)std::max(1LL, std::min({want, n_pairs, (long long)UINT32_MAX}));
       VD_HIP(ctx->rec_meta.ensure(cap), "alloc records");
       VD_HIP(ctx->rec_tris.ensure((size_t)cap * vd::rec_stride(fast_tcap)), "alloc records");
@@ -1429,6 +1440,7 @@ namespace vdi {
 
 hipStream_t stream(vd_ctx* ctx) { return ctx->stream; }
 void set_error(vd_ctx* ctx, const char* msg) { ctx->err = msg; }
+void limit_records(vd_ctx* ctx, long long more) { ctx->more_records = more; }
 
 int assemble(vd_ctx* ctx, const JobDev* jobs, int n) {
   if (!ctx || !jobs || n < 1) return VD_ERR_ARG;

@@ -46,6 +46,15 @@ void set_error(vd_ctx* ctx, const char* msg);
 // 4.65 per tet at a tenth as many sites (counted: 4.60 at 998,250 tets, 4.65
 // at 146,334), growing as the cells shrink against the tets.
 double pieces_estimate(double n_tets, double n_sites);
+// Volume-pass records per tet that the automatic buffer holds at TK candidates
+// per tet: a tenth of the pairs, and at least 1.3 times the estimated pieces
+// (the tenth alone held 2 per tet at the heuristic's TK = 20, and the pieces
+// past it were integrated inside the clipping, or with the robust moments
+// re-clipped: 1.42 -> 1.10 ms and 2.0 -> 1.05 ms per clipping at 146,334 tets,
+// 16.8 -> 5.9 ms at 998,250).
+double records_per_tet(double n_tets, double n_sites, int TK);
+// At most `more` records beyond a tenth of the pairs in the automatic buffer.
+void limit_records(vd_ctx* ctx, long long more);
 // Vertex cap of the site-major launch under configuration c (its site_tcap,
 // or the automatic choice).
 int site_tcap_of(const vd_config& c);

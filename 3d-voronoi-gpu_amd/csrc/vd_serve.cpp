@@ -328,6 +328,10 @@ int vd_server_step(vd_server* s, int* n_running, int* n_pending) {
       const std::vector<vdi::JobDev> cur = s->devs(s->running);
       int rc = vdi::assemble(s->ctx, cur.data(), (int)cur.size());
       if (rc != VD_OK) return s->fail(rc, vd_ctx_error(s->ctx));
+      // the jobs' footprints count one volume-pass record per ten pairs; more
+      // only from what the budget has left
+      vdi::limit_records(s->ctx, (long long)((s->budget - s->used) /
+                                             (16 + 4 * (size_t)vd::rec_stride(vdi::site_tcap_of(s->cfg)))));
       s->assembled = s->running;
       s->changed = false;
     }

@@ -45,3 +45,19 @@ def test_small_problem_caps(vdn, O, n, ns):
             e.knn_step()
             e.clip_step()
             np.testing.assert_array_equal(e.moments(), r["site_vals"])
+
+
+@pytest.mark.parametrize("n,ns,tk", [(22, 6389, 20), (12, 9000, 20), (8, 3000, 64)])
+def test_records_at_few_candidates(vdn, O, n, ns, tk):
+    """More pieces than a tenth of the pairs (few candidates, dense sites)."""
+    verts, tets, sites = problem("cube", n, ns)
+    sk, tkn = oracle_knn("cube", n, ns, 90, tk)
+    for moments in ("reference", "robust"):
+        r = O.clip_tets(sites, sk, verts, tets, tkn, geom="f32", pair_acc="f64", site_mode=O.SITE_FIXED,
+                        moments=moments, want_pairs=False)
+        with vdn.Engine(tet_k=tk, accum="f64", moments=moments) as e:
+            e.set_mesh(verts, tets)
+            e.set_sites(sites)
+            e.knn_step()
+            e.clip_step()
+            np.testing.assert_array_equal(e.moments(), r["site_vals"])
