@@ -58,9 +58,10 @@ __device__ __forceinline__ uint32_t xor_lane32(uint32_t v, int j, int lane) {
     case 1: return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0xB1, 0xF, 0xF, false);   // quad_perm [1,0,3,2]
     case 2: return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x4E, 0xF, 0xF, false);   // quad_perm [2,3,0,1]
     case 4: {
-      const int from_below = __builtin_amdgcn_mov_dpp(x, 0x124, 0xF, 0xF, false);  // row_ror:4, lane i - 4
-      const int from_above = __builtin_amdgcn_mov_dpp(x, 0x12C, 0xF, 0xF, false);  // row_ror:12, lane i + 4
-      return (uint32_t)((lane & 4) ? from_below : from_above);
+      // lanes without bit 2 (banks 0 and 2 of a row): row_ror:12, lane i + 4;
+      // then the others (banks 1 and 3): row_ror:4, lane i - 4
+      const int from_above = __builtin_amdgcn_mov_dpp(x, 0x12C, 0xF, 0x5, false);
+      return (uint32_t)__builtin_amdgcn_update_dpp(from_above, x, 0x124, 0xF, 0xA, false);
     }
     case 8: return (uint32_t)__builtin_amdgcn_mov_dpp(x, 0x128, 0xF, 0xF, false);  // row_ror:8
     default: return bperm32(v, lane ^ j);
@@ -118,12 +119,43 @@ __device__ __forceinline__ int batch_owner(int* mark, int lane, int cnt, int exc
   return own;
 }
 __device__ __forceinline__ uint64_t umin64(uint64_t a, uint64_t b) { return a < b ? a : b; }
-__device__ __forceinline__ uint64_t umax64(uint64_t a, uint64_t b) { return a < b ? b : a; }
 
-__device__ __forceinline__ uint64_t knn_key(float d2, uint32_t id) {
-  return ((uint64_t)__float_as_uint(d2) << 32) | id;
+// A key orders by (d2, id): the bits of d2 >= 0 (every NaN taken as the same
+// one, after infinity) plus kKeyShift in the high word, the id in the low one.
+// As a double it is positive, finite and normal (the shift lifts it out of the
+// subnormals, and the largest high word, of a NaN, is below the exponent of
+// infinity), so the order of the keys is the order of the doubles, and one
+// v_min_f64 takes the smaller of two keys unchanged where a 64-bit integer
+// compare needs two selects after it.  kNoKey, larger than every key, is an
+// empty place.
+constexpr uint32_t kKeyShift = 0x00100000u;
+constexpr uint64_t kNoKey = 0x7FEFFFFFFFFFFFFFull;
+__device__ __forceinline__ uint32_t key_word(float d2) { return min(__float_as_uint(d2), 0x7FC00000u) + kKeyShift; }
+__device__ __forceinline__ uint64_t knn_key(float d2, uint32_t id) { return ((uint64_t)key_word(d2) << 32) | id; }
+// The largest key at distance d2.
+__device__ __forceinline__ uint64_t key_bound(float d2) { return ((uint64_t)key_word(d2) << 32) | 0xffffffffull; }
+__device__ __forceinline__ float key_d2(uint64_t k) { return __uint_as_float((uint32_t)(k >> 32) - kKeyShift); }
+
+// min(a, b), max(a, b) and min(a, -b) of keys and negated keys (sign bit set).
+// The s_nop is the distance that a VALU result needs before a DPP move reads
+// it, which the compiler does not add behind inline assembly.
+__device__ __forceinline__ uint64_t key_min(uint64_t a, uint64_t b) {
+  uint64_t r;
+  asm("v_min_f64 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
 }
-__device__ __forceinline__ float key_d2(uint64_t k) { return __uint_as_float((uint32_t)(k >> 32)); }
+__device__ __forceinline__ uint64_t key_max(uint64_t a, uint64_t b) {
+  uint64_t r;
+  asm("v_max_f64 %0, %1, %2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+__device__ __forceinline__ uint64_t key_min_neg(uint64_t a, uint64_t b) {
+  uint64_t r;
+  asm("v_min_f64 %0, %1, -%2\n\ts_nop 1" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+// x with its sign bit flipped where `sign` (0 or 0x80000000) says so.
+__device__ __forceinline__ uint64_t flip(uint64_t x, uint32_t sign) { return x ^ ((uint64_t)sign << 32); }
 
 __device__ __forceinline__ float dist2(const float4& r, const float4& q) {
   const float dx = r.x - q.x, dy = r.y - q.y, dz = r.z - q.z;
@@ -490,51 +522,67 @@ struct TopK {
   uint64_t s[M];
 };
 
-// Bitonic sort of one key per lane across the wave, ascending.
-__device__ __forceinline__ uint64_t wave_sort64(uint64_t x, int lane) {
+// The sorting networks keep a lane's key negated where the lane takes the
+// larger key of its pair: with partner's value o, which has the other sign,
+// min(x, -o) is then the step for both lanes of a pair, one instruction after
+// the move, and the sign flips between two steps by a mask that the lane
+// number gives (two compares and six selects per step without it; kNN phase
+// at 1M tets / 100,000 sites 1.84 -> 1.56 ms).
+//
+// Sign bit of bit i of the lane number.
+__device__ __forceinline__ uint32_t lane_sign(int lane, int i) { return ((uint32_t)lane << (31 - i)) & 0x80000000u; }
+
+// Bitonic sort of one key per lane across the wave, ascending, or descending
+// with desc = 0x80000000 (wave-uniform).  In the step (k, j) the lanes whose
+// bits j and k differ take the larger key.
+__device__ __forceinline__ uint64_t wave_sort64(uint64_t x, int lane, uint32_t desc) {
+  x = flip(x, lane_sign(lane, 0) ^ lane_sign(lane, 1) ^ desc);
 #pragma unroll
-  for (int k = 2; k <= 64; k <<= 1) {
+  for (int k = 1; k <= 6; ++k) {
 #pragma unroll
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      const uint64_t o = xor_lane64(x, j, lane);
-      const bool up = (lane & k) == 0;
-      const bool lower = (lane & j) == 0;
-      x = (lower == up) ? umin64(x, o) : umax64(x, o);
+    for (int j = k - 1; j >= 0; --j) {
+      x = key_min_neg(x, xor_lane64(x, 1 << j, lane));
+      if (j > 0)
+        x = flip(x, lane_sign(lane, j) ^ lane_sign(lane, j - 1));
+      else if (k < 5)
+        x = flip(x, lane_sign(lane, 0) ^ lane_sign(lane, k + 1));
+      else if (k == 5)
+        x = flip(x, lane_sign(lane, 0));
     }
   }
-  return x;
+  return flip(x, lane_sign(lane, 0) ^ desc);
 }
 
 // Sorted merge of 64 new keys (one per lane) into the top list; into an
 // empty list (first) the sorted keys are the list.
 template <int M>
 __device__ __forceinline__ void topk_merge(TopK<M>& L, uint64_t x, int lane, bool first = false) {
-  x = wave_sort64(x, lane);
+  x = wave_sort64(x, lane, first ? 0u : 0x80000000u);
   if (first) {
     L.s[0] = x;
     return;
   }
-  // min against the reversed batch gives the 64*M smallest as a bitonic sequence
-  const uint64_t r = bperm64(x, 63 - lane);
-  L.s[M - 1] = umin64(L.s[M - 1], r);
+  // min against the descending batch gives the 64*M smallest as a bitonic sequence
+  L.s[M - 1] = key_min(L.s[M - 1], x);
 #pragma unroll
   for (int js = M / 2; js >= 1; js >>= 1) {
 #pragma unroll
     for (int s = 0; s < M; ++s) {
       if ((s & js) == 0) {
         const uint64_t a = L.s[s], b = L.s[s + js];
-        L.s[s] = umin64(a, b);
-        L.s[s + js] = umax64(a, b);
+        L.s[s] = key_min(a, b);
+        L.s[s + js] = key_max(a, b);
       }
     }
   }
 #pragma unroll
-  for (int j = 32; j > 0; j >>= 1) {
-    const bool lower = (lane & j) == 0;
+  for (int s = 0; s < M; ++s) L.s[s] = flip(L.s[s], lane_sign(lane, 5));
+#pragma unroll
+  for (int j = 5; j >= 0; --j) {
 #pragma unroll
     for (int s = 0; s < M; ++s) {
-      const uint64_t o = xor_lane64(L.s[s], j, lane);
-      L.s[s] = lower ? umin64(L.s[s], o) : umax64(L.s[s], o);
+      const uint64_t m = key_min_neg(L.s[s], xor_lane64(L.s[s], 1 << j, lane));
+      L.s[s] = flip(m, j > 0 ? lane_sign(lane, j) ^ lane_sign(lane, j - 1) : lane_sign(lane, 0));
     }
   }
 }
@@ -660,7 +708,7 @@ constexpr int kUnionCap = VD_KNN_UNION_CAP;
 // At most this many keys staged after the last merge are inserted one at a
 // time instead of sorted and merged.
 #ifndef VD_KNN_INSERT_MAX
-#define VD_KNN_INSERT_MAX 12
+#define VD_KNN_INSERT_MAX 6
 #endif
 constexpr int kInsertMax = VD_KNN_INSERT_MAX;
 
@@ -836,20 +884,20 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
 
   TopK<M> L;
 #pragma unroll
-  for (int s = 0; s < M; ++s) L.s[s] = ~0ull;
-  uint64_t bound = ~0ull;
+  for (int s = 0; s < M; ++s) L.s[s] = kNoKey;
+  uint64_t bound = kNoKey;
   if (prev_r >= 0.f && prev_inst == inst) {
     const float dx = qp.x - prev_qp.x, dy = qp.y - prev_qp.y, dz = qp.z - prev_qp.z;
     const float b = prev_r + sqrtf(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
     const float b2 = b * b * (1.f + 1e-5f);
-    if (b2 < INFINITY) bound = ((uint64_t)__float_as_uint(b2) << 32) | 0xffffffffull;
+    if (b2 < INFINITY) bound = key_bound(b2);
   }
   if (from_list) {
     // the bound the list was gathered for: r0 + |q - q0|
     const float dx = qp.x - q0p.x, dy = qp.y - q0p.y, dz = qp.z - q0p.z;
     const float b = r0 + sqrtf(fmaf(dz, dz, fmaf(dy, dy, dx * dx)));
     const float b2 = b * b * (1.f + 1e-5f);
-    bound = umin64(bound, ((uint64_t)__float_as_uint(b2) << 32) | 0xffffffffull);
+    bound = umin64(bound, key_bound(b2));
   }
   if (use_hint) {
     // the query's previous result: its k points' current distances
@@ -858,7 +906,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       const int lo = a.pt_begin ? a.pt_begin[inst] : 0, hi = a.pt_begin ? a.pt_begin[inst + 1] : a.n_ref;
       hb = hint_bound<M>(a, out_row, qp, self, lo, hi, lane);
     }
-    if (hb >= 0.f) bound = umin64(bound, ((uint64_t)__float_as_uint(hb) << 32) | 0xffffffffull);
+    if (hb >= 0.f) bound = umin64(bound, key_bound(hb));
   }
   uint64_t thr = bound;
   int staged = 0;
@@ -873,7 +921,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
     wave_sync();
     if (staged >= 64) {
       const uint64_t x = stage[lane];
-      const uint64_t rest = (lane + 64 < staged) ? stage[lane + 64] : ~0ull;
+      const uint64_t rest = (lane + 64 < staged) ? stage[lane + 64] : kNoKey;
       wave_sync();
       if (lane + 64 < staged) stage[lane] = rest;
       staged -= 64;
@@ -887,7 +935,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
   if (from_list) {
     for (int f0 = 0; f0 < n_uni; f0 += 64) {
       const int f = f0 + lane;
-      uint64_t key = ~0ull;
+      uint64_t key = kNoKey;
       bool ok = false;
       if (f < n_uni) {
         const float4 p = uni[f];
@@ -904,7 +952,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
     // offsets are sorted by lb: once the first of the batch is beyond the k-th
     // distance, so are all later ones
     const float lbd = fmaxf(0.f, sqrtf((float)a.offsets[ob].w) * g.h - 2.f * g.slack);
-    if (thr != ~0ull && lbd * lbd * (1.f - 1e-5f) > kth) {
+    if (thr != kNoKey && lbd * lbd * (1.f - 1e-5f) > kth) {
       done = true;
       break;
     }
@@ -914,7 +962,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       const int4 o = a.offsets[oi];
       const int cx = qc[0] + o.x, cy = qc[1] + o.y, cz = qc[2] + o.z;
       if (cx >= 0 && cx < g.dim[0] && cy >= 0 && cy < g.dim[1] && cz >= 0 && cz < g.dim[2]) {
-        if (thr == ~0ull || !(cell_bound(g, qp, cx, cy, cz) > kth)) {
+        if (thr == kNoKey || !(cell_bound(g, qp, cx, cy, cz) > kth)) {
           const int c = cbase + cx + g.dim[0] * (cy + g.dim[1] * cz);
           st = a.start[c];
           cnt = a.start[c + 1] - st;
@@ -930,7 +978,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       const int f = f0 + lane;
       const int own = batch_owner(mark, lane, cnt, excl, f0, carry);
       const int o_st = __shfl(st, own), o_ex = __shfl(excl, own);
-      uint64_t key = ~0ull;
+      uint64_t key = kNoKey;
       bool ok = false;
       if (f < total) {
         const int idx = o_st + (f - o_ex);
@@ -948,7 +996,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
     const int r0 = a.start[cbase], r1 = a.start[cbase + g.ncell];
     for (int f0 = r0; f0 < r1; f0 += 64) {
       const int f = f0 + lane;
-      uint64_t key = ~0ull;
+      uint64_t key = kNoKey;
       bool ok = false;
       if (f < r1) {
         // skip cells already visited: those inside the offset table's reach
@@ -974,14 +1022,14 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       }
     }
   } else if (staged > 0) {
-    const uint64_t x = lane < staged ? stage[lane] : ~0ull;
+    const uint64_t x = lane < staged ? stage[lane] : kNoKey;
     topk_merge<M>(L, x, lane, empty);
   }
 #pragma unroll
   for (int s = 0; s < M; ++s) {
     const int j = s * 64 + lane;
     if (j < a.k) {
-      const int32_t id = L.s[s] == ~0ull ? -1 : (int32_t)(uint32_t)L.s[s];
+      const int32_t id = L.s[s] == kNoKey ? -1 : (int32_t)(uint32_t)L.s[s];
       if (a.out_pitch > 0)
         a.out[(long long)j * a.out_pitch + out_row] = id;
       else
@@ -989,7 +1037,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
     }
   }
   const uint64_t kth = topk_kth<M>(L, a.k);
-  prev_r = kth == ~0ull ? -1.f : sqrtf(key_d2(kth));
+  prev_r = kth == kNoKey ? -1.f : sqrtf(key_d2(kth));
   prev_qp = qp;
   prev_inst = inst;
 
