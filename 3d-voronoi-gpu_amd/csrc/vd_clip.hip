@@ -933,6 +933,15 @@ __device__ __forceinline__ void count_status(const ClipArgs& a, int status, bool
 
 __device__ __forceinline__ P4 site_at(const ClipArgs& a, int i) { return ld4(a.sites, i); }
 
+// Tet of a pair: pair / TK (Granlund and Montgomery's division by an invariant
+// integer with the constants of set_tk; the compiler's division by a run-time
+// value takes some 20 instructions).
+__device__ __forceinline__ unsigned tet_of(const ClipArgs& a, unsigned pair) {
+  if (a.tk_mul == 0u) return pair >> a.tk_shift;
+  const unsigned t = __umulhi(a.tk_mul, pair);
+  return (t + ((pair - t) >> 1)) >> a.tk_shift;
+}
+
 __device__ __forceinline__ void tet_corners(const ClipArgs& a, int t, P4 v[4]) {
   const float4* r = a.tet_xyz + 3 * (size_t)t;
   corners_of(r[0], r[1], r[2], v);
@@ -1249,7 +1258,6 @@ __global__ __launch_bounds__(64) void k_clip_plain(ClipArgs a) {
 constexpr int kQueue = 128;           // ring of queued pair ids
 constexpr float kInvalidNbr = -1.f;   // table mark of an out-of-range neighbour id
 constexpr int kIdle = 0, kClipping = 1;  // lane states
-constexpr int kRecChunk = 128;           // record slots a wave reserves at a time
 // Records of polytopes with more than kRecSplit vertices go to chunks of their
 // own, so that a wave of the volume pass (64 records of one chunk) runs over
 // polytopes of similar size.
@@ -1381,7 +1389,7 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
       pslot = qp < qsplit ? feed_slot ^ 1 : feed_slot;
       pv = 0;
       lst = kClipping;
-      ptet = ppair / (unsigned)a.TK;
+      ptet = tet_of(a, ppair);
       c.ps.bis = bis + pslot * K4;
       c.init_tet_prep(site_at(a, pslot ? site1 : site0), a.tet_prep + kTetPrepWords * (size_t)ptet);
     }
@@ -1551,7 +1559,7 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
       }
     }
     // (4) records of the polytopes for the volume pass, one slot per
-    // deferring lane, from slots the wave reserves kRecChunk at a time (one
+    // deferring lane, from slots the wave reserves rec_chunk at a time (one
     // global counter shared by every wave would serialise them)
     const unsigned long long dm = __ballot(defer);
     if (dm != 0) {
@@ -1573,11 +1581,11 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
           } else {
             const int leader = __builtin_ctzll(m);
             unsigned base = 0;
-            if (lane == leader) base = atomicAdd(a.rec_count, (unsigned)kRecChunk);
+            if (lane == leader) base = atomicAdd(a.rec_count, a.rec_chunk);
             base = __shfl(base, leader);
             if (mine) slot = rk < have ? next + rk : base + (rk - have);
             next = base + (need - have);
-            end = base + (unsigned)kRecChunk;
+            end = base + a.rec_chunk;
           }
         };
         reserve(dm0, rec_next0, rec_end0);
@@ -1615,34 +1623,57 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
 }
 
 // Emptiness test of the site-major form as a pass of its own, before the
-// clipping: one wavefront per site builds the site's first `depth` bisectors
-// as the clipping's tables hold them, tests the site's pairs 64 at a time
-// (all four tet corners beyond one of them by more than the FP32 rounding
-// bound plus kCullMargin, with the early exit once the tet's nearest corner
-// is within |z - s| / 2 of the seed) and compacts the survivors, in their
-// order, to the front of the site's pair range; pair_count[s] gets their
-// number.  Small and without polytope state, it runs at full occupancy, where
-// inside the clipping kernel the same test ran at under two waves per SIMD.
+// clipping.  A workgroup takes a site: one wavefront, or four on small problems
+// (a site has several hundred pairs, which one wave tests in a dozen trips).
+// It holds the site's first `depth` bisectors in LDS as planes n.x + w >= 0 on
+// the seed's side, each w raised by the test's margin: a tet whose four corners
+// all evaluate below zero lies beyond the bisector by more than the rounding
+// bound plus kCullMargin and its pair is empty.
+//
+// Which bisector empties a pair depends on where the tet lies: for each of the
+// 26 directions of a 3x3x3 neighbourhood the wave picks the two bisectors whose
+// sites are nearest to the point that far out, and a pair is tested against the
+// two of its centroid's direction first, 64 pairs at a time.  That decides 86 %
+// of the pairs (all 16 bisectors empty 89 %; counted at 48,000 tets / 4,800
+// sites, tet_k 64; the two nearest sites alone 45 %).  The rest are queued and
+// tested against every bisector 64 at a time, up to the first whose half
+// distance reaches the tet's nearest corner (no later one can succeed, the
+// distances do not decrease).  Survivors are compacted to the front of the
+// site's range, in pair_ids itself (one wave, which has read what it
+// overwrites) or in out_ids, and their number goes to pair_count.
+//
+// Testing each pair against the bisectors in list order was bound by VALU
+// issue: 335 instructions per 64 pairs and 545 us at 1M tets / 100,000 sites
+// (64M pairs); this takes 178 and 393 us.  The corners of the next 64 pairs are
+// loaded while these are tested (455 us without).
 constexpr int kCullMaxDepth = 256;
 constexpr int kXcds = 8;  // MI355X: accelerator complex dies, one L2 each
+constexpr int kCullQueue = 128;
 
-// Pairs per lane per trip of the emptiness pass: one (a lane's loop runs
-// until every pair it holds is decided, so two per lane left more lanes idle:
-// 0.05 ms slower per iteration at 1M tets, four 0.12 ms).
-constexpr int kCullPairs = 1;
-__device__ __forceinline__ bool any_open(const bool* o) {
-  bool r = false;
-#pragma unroll
-  for (int h = 0; h < kCullPairs; ++h) r = r || o[h];
-  return r;
+// The wave's LDS writes before its reads after (the lanes run in step).
+__device__ __forceinline__ void wave_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  __builtin_amdgcn_wave_barrier();
 }
 
-__global__ __launch_bounds__(64) void k_cull_site(ClipArgs a, int depth, unsigned* pair_ids, unsigned* pair_count) {
+__device__ __forceinline__ bool beyond(const float4& e, const P4 v[4]) {
+  float hi = -INFINITY;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) hi = fmaxf(hi, fmaf(e.z, v[k].z, fmaf(e.y, v[k].y, fmaf(e.x, v[k].x, e.w))));
+  return hi < 0.f;
+}
+
+template <int W>
+__global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, const unsigned* pair_ids,
+                                                      unsigned* out_ids, unsigned* pair_count) {
   extern __shared__ __align__(16) uint8_t smem[];
-  float4* eb = (float4*)smem;   // [depth] bisector (n, w)
-  float4* ec = eb + depth;      // [depth] |z - s|^2, |n|_1, |w|, kCullMargin * |n|
-  const int lane = threadIdx.x;
-  unsigned n_culled = 0;  // over the block's sites: one histogram atomic per block
+  float4* eb = (float4*)smem;            // [depth] bisector (n, w + margin)
+  float* dd = (float*)(eb + depth);      // [depth] |z - s|^2
+  uint32_t* first2 = (uint32_t*)(dd + depth);    // [27] the direction's two bisectors
+  unsigned* survivors = (unsigned*)(first2 + 27);  // their number so far
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  unsigned* queue = survivors + 1 + wv * kCullQueue;  // [kCullQueue] the wave's ring of undecided pairs
+  unsigned n_culled = 0;  // over the wave's pairs: one histogram atomic per wave
   // Blocks go to the 8 XCDs in turn, each with an L2 of its own: the blocks of
   // one XCD take one contiguous stretch of the site order, so that the tets
   // that nearby sites share are fetched into the same L2.
@@ -1653,7 +1684,7 @@ __global__ __launch_bounds__(64) void k_cull_site(ClipArgs a, int depth, unsigne
     const int s = a.site_order ? a.site_order[si] : si;
     const unsigned pb = a.pair_start[s], pe = a.pair_start[s + 1];
     if (pb == pe) {
-      if (lane == 0) pair_count[s] = 0;
+      if (threadIdx.x == 0) pair_count[s] = 0;
       continue;
     }
     // Cell form: no cell (every pair of the site takes the cell's status), or
@@ -1664,101 +1695,143 @@ __global__ __launch_bounds__(64) void k_cull_site(ClipArgs a, int depth, unsigne
     // the overflow.  Every pair is kept.
     if (a.cell_status && ((a.cell_status[s] != kSuccess && a.cell_status[s] != kSecurityRadiusNotReached) ||
                           a.cell_nv[s] + 4 > a.pcap || a.cell_nt[s] + 6 >= a.tcap)) {
-      if (lane == 0) pair_count[s] = pe - pb;
+      if (threadIdx.x == 0) pair_count[s] = pe - pb;
+      if (W > 1)
+        for (unsigned i = pb + threadIdx.x; i < pe; i += 64 * W) out_ids[i] = pair_ids[i];
       continue;
     }
     const P4 sp = site_at(a, s);
     const int32_t* nbr = a.site_knn + (size_t)s * a.K;
+    // pair ids are read two trips ahead and tet corners one
+    auto pair_at = [&](unsigned i) { return i < pe ? pair_ids[i] : 0u; };
+    unsigned c0 = pb + 64 * wv;
+    unsigned pair = pair_at(c0 + lane), pair1 = pair_at(c0 + 64 * W + lane);
     __syncthreads();  // the previous site's readers are done
-    for (int v = lane; v < depth; v += 64) {
-      const int z = nbr[v];
-      if ((unsigned)z >= (unsigned)a.n_sites) {
-        eb[v] = make_float4(0.f, 0.f, 0.f, 0.f);
-        ec[v] = make_float4(kInvalidNbr, 0.f, 0.f, 0.f);
-        continue;
+    int dv = depth;  // bisectors before the first invalid neighbour, which ends the clipping there
+    for (int v0 = 0; v0 < depth; v0 += 64) {
+      const int v = v0 + lane;
+      const int z = v < depth ? nbr[v] : 0;
+      const bool bad = (unsigned)z >= (unsigned)a.n_sites;
+      const unsigned long long m = __ballot(bad);
+      if (m && dv == depth) dv = v0 + __builtin_ctzll(m);
+      if (v < depth && !bad && wv == 0) {
+        const P4 zp = site_at(a, z);
+        const P4 eq = bisector(sp, zp);
+        const P4 d = sub3(zp, sp);
+        const float d2 = dot3(d, d);
+        // the rounding of the evaluation (relative kCullRound of |n|_1 max|x| +
+        // |w|: one rounding of w and the margin, three of partial sums, all
+        // bounded by about that) plus kCullMargin in distance, times |n|
+        const float margin = fmaf(kCullRound, fmaf(fabsf(eq.x) + fabsf(eq.y) + fabsf(eq.z), a.max_coord, fabsf(eq.w)),
+                                  kCullMargin * __builtin_amdgcn_sqrtf(d2));
+        eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w + margin);
+        dd[v] = d2;
       }
-      const P4 zp = site_at(a, z);
-      const P4 eq = bisector(sp, zp);
-      const P4 d = sub3(zp, sp);
-      const float dd = dot3(d, d);
-      eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w);
-      ec[v] = make_float4(dd, fabsf(eq.x) + fabsf(eq.y) + fabsf(eq.z), fabsf(eq.w), kCullMargin * __builtin_amdgcn_sqrtf(dd));
+    }
+    if (threadIdx.x == 0) *survivors = 0u;
+    P4 v[4];
+    tet_corners(a, (int)tet_of(a, pair), v);  // (pair 0's past the range)
+    __syncthreads();
+    if (threadIdx.x < 27 && dv > 0) {
+      const float ux = (float)(lane % 3 - 1), uy = (float)(lane / 3 % 3 - 1), uz = (float)(lane / 9 - 1);
+      const float r = 2.f * __builtin_amdgcn_sqrtf(dd[dv - 1] / fmaxf(1.f, ux * ux + uy * uy + uz * uz));
+      // |s + R u - z|^2 = R^2 - 2 R u.(z - s) + |z - s|^2, and z - s = -n
+      int q0 = 0, q1 = 0;
+      float s0 = INFINITY, s1 = INFINITY;
+#pragma unroll 4
+      for (int q = 0; q < dv; ++q) {
+        const float4 e = eb[q];
+        const float sc = fmaf(r, fmaf(uz, e.z, fmaf(uy, e.y, ux * e.x)), dd[q]);
+        if (sc < s0) {
+          s1 = s0;
+          q1 = q0;
+          s0 = sc;
+          q0 = q;
+        } else if (sc < s1) {
+          s1 = sc;
+          q1 = q;
+        }
+      }
+      first2[lane] = (uint32_t)q0 | ((uint32_t)q1 << 16);
     }
     __syncthreads();
-    unsigned w = pb;
-    // kCullPairs pairs per lane per trip (c0 + lane, c0 + 64 + lane, ...)
-    for (unsigned c0 = pb; c0 < pe; c0 += 64 * kCullPairs) {
-      unsigned pair[kCullPairs];
-      bool live[kCullPairs], culled[kCullPairs] = {}, open[kCullPairs];
-      P4 v[kCullPairs][4] = {};
-      float pmax[kCullPairs] = {}, vmin2[kCullPairs] = {};
-#pragma unroll
-      for (int h = 0; h < kCullPairs; ++h) {
-        const unsigned i = c0 + 64 * h + lane;
-        live[h] = i < pe;
-        pair[h] = live[h] ? pair_ids[i] : 0u;
+    unsigned w = pb, qhead = 0, qtail = 0;  // w: one wave's next place
+    auto record = [&](unsigned pair, bool culled) {
+      if (culled && a.pair_status) a.pair_status[pair] = (uint8_t)kNoIntersection;
+      if (culled && a.pair_vals) {
+        double* pvals = a.pair_vals + 4 * (size_t)pair;
+        pvals[0] = pvals[1] = pvals[2] = pvals[3] = 0.0;
       }
+      n_culled += (unsigned)__popcll(__ballot(culled));
+    };
+    auto rank = [](unsigned long long m) {
+      return (unsigned)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0));
+    };
+    // the first n queued pairs against every bisector; the survivors to the
+    // front of the range (one wave: every position written here has been read,
+    // as w never passes the pairs read so far)
+    auto finish = [&](unsigned n) {
+      const bool live = (unsigned)lane < n;
+      const unsigned pr = live ? queue[(qhead + lane) % kCullQueue] : 0u;
+      P4 t[4];
+      tet_corners(a, (int)tet_of(a, pr), t);
+      float vmin2 = INFINITY;
 #pragma unroll
-      for (int h = 0; h < kCullPairs; ++h)
-        if (live[h]) tet_corners(a, (int)(pair[h] / (unsigned)a.TK), v[h]);
-#pragma unroll
-      for (int h = 0; h < kCullPairs; ++h) {
-        open[h] = live[h];
-        if (live[h]) {
-          vmin2[h] = INFINITY;
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            pmax[h] = fmaxf(pmax[h], fmaxf(fabsf(v[h][j].x), fmaxf(fabsf(v[h][j].y), fabsf(v[h][j].z))));
-            const P4 d = sub3(v[h][j], sp);
-            vmin2[h] = fminf(vmin2[h], dot3(d, d));
-          }
-        }
+      for (int k = 0; k < 4; ++k) {
+        const P4 d = sub3(t[k], sp);
+        vmin2 = fminf(vmin2, dot3(d, d));
       }
-      for (int q = 0; q < depth && any_open(open); ++q) {
-        const float4 f = ec[q];
-        const float4 e = eb[q];
-        // rounding bound of the plane evaluation (relative kCullRound of
-        // |n|_1 * max|x| + |w|: three roundings of partial sums bounded by
-        // that) plus the required depth beyond the plane (kCullMargin in
-        // distance, times |n|)
-        // (as selects: a pair's loads are in flight together and every lane
-        // runs the same instructions)
-#pragma unroll
-        for (int h = 0; h < kCullPairs; ++h) {
-          // an invalid neighbour ends the clipping there; and once the tet's
-          // nearest corner is within |z - s| / 2 of the seed it is on the
-          // seed's side of this bisector and of every later one (the
-          // neighbour distances do not decrease)
-          const bool stop = f.x == kInvalidNbr || 4.f * vmin2[h] <= f.x;
-          const float lim = -fmaf(kCullRound, fmaf(f.y, pmax[h], f.z), f.w);
-          float hi = -INFINITY;
-#pragma unroll
-          for (int k = 0; k < 4; ++k)
-            hi = fmaxf(hi, fmaf(e.z, v[h][k].z, fmaf(e.y, v[h][k].y, fmaf(e.x, v[h][k].x, e.w))));
-          const bool cut = open[h] && !stop && hi < lim;
-          culled[h] = culled[h] || cut;
-          open[h] = open[h] && !stop && !cut;
-        }
+      bool open = live, culled = false;
+      for (int q = 0; q < dv && __ballot(open) != 0; ++q) {
+        const bool cut = open && beyond(eb[q], t);
+        culled = culled || cut;
+        open = open && !cut && !(4.f * vmin2 <= dd[q]);
       }
-#pragma unroll
-      for (int h = 0; h < kCullPairs; ++h) {
-        if (culled[h] && a.pair_status) a.pair_status[pair[h]] = (uint8_t)kNoIntersection;
-        if (culled[h] && a.pair_vals) {
-          double* pvals = a.pair_vals + 4 * (size_t)pair[h];
-          pvals[0] = pvals[1] = pvals[2] = pvals[3] = 0.0;
-        }
-        n_culled += (unsigned)__popcll(__ballot(culled[h]));
-        // survivors to the front, in order: every position written here has
-        // been read (w never passes the pairs read so far)
-        const bool keep = live[h] && !culled[h];
-        const unsigned long long mask = __ballot(keep);
-        const unsigned below =
-            (unsigned)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0));
-        if (keep) pair_ids[w + below] = pair[h];
-        w += (unsigned)__popcll(mask);
+      record(pr, culled);
+      const unsigned long long keep = __ballot(live && !culled);
+      const unsigned kept = (unsigned)__popcll(keep);
+      if (W > 1 && kept) {
+        unsigned at = 0;
+        if (lane == 0) at = atomicAdd(survivors, kept);
+        w = pb + (unsigned)__builtin_amdgcn_readfirstlane((int)at);
       }
+      if (live && !culled) out_ids[w + rank(keep)] = pr;
+      w += kept;
+      qhead += n;
+    };
+    for (; c0 < pe; c0 += 64 * W) {
+      const bool live = c0 + lane < pe;
+      const unsigned cur = pair;
+      bool culled = false;
+      if (dv > 0) {
+        // direction of the centroid: per axis -1, 0 or 1, where 0 is less than
+        // tan(22.5 deg) of the largest component
+        const float cx = fmaf(-4.f, sp.x, (v[0].x + v[1].x) + (v[2].x + v[3].x));
+        const float cy = fmaf(-4.f, sp.y, (v[0].y + v[1].y) + (v[2].y + v[3].y));
+        const float cz = fmaf(-4.f, sp.z, (v[0].z + v[1].z) + (v[2].z + v[3].z));
+        const float t = 0.41421356f * fmaxf(fabsf(cx), fmaxf(fabsf(cy), fabsf(cz)));
+        const int dir = 13 + (cx > t) - (cx < -t) + 3 * ((cy > t) - (cy < -t)) + 9 * ((cz > t) - (cz < -t));
+        const uint32_t f = first2[dir];
+        const bool b0 = beyond(eb[f & 0xffffu], v), b1 = beyond(eb[f >> 16], v);
+        culled = live && (b0 || b1);
+      }
+      pair = pair1;
+      tet_corners(a, (int)tet_of(a, pair), v);
+      pair1 = pair_at(c0 + 128 * W + lane);
+      record(cur, culled);
+      const unsigned long long undecided = __ballot(live && !culled);
+      if (live && !culled) queue[(qtail + rank(undecided)) % kCullQueue] = cur;
+      qtail += (unsigned)__popcll(undecided);
+      wave_fence();
+      if (qtail - qhead >= 64u) finish(64u);
     }
-    if (lane == 0) pair_count[s] = w - pb;
+    if (qtail != qhead) finish(qtail - qhead);
+    if (W > 1) {
+      __syncthreads();
+      if (threadIdx.x == 0) pair_count[s] = *survivors;
+    } else if (lane == 0) {
+      pair_count[s] = w - pb;
+    }
   }
   if (lane == 0 && a.status_hist && n_culled) add_status(a, kNoIntersection, n_culled);
 }
@@ -2160,7 +2233,7 @@ __global__ __launch_bounds__(64) void k_cells_clip(ClipArgs a, CellStore cs, int
     int status = kNoIntersection;
     if (live) {
       P4 v[4];
-      tet_corners(a, (int)(pair / (unsigned)a.TK), v);
+      tet_corners(a, (int)tet_of(a, pair), v);
       c.ps.cpl = cpl + sl * a.pcap;
       c.ps.nvc = cnv;
       c.seed = site_at(a, s);
@@ -2261,7 +2334,7 @@ __global__ __launch_bounds__(64) void k_cells_clip(ClipArgs a, CellStore cs, int
       bool culled = false;
       if (live && a.cull_depth > 0 && may_skip) {
         P4 v[4];
-        tet_corners(a, (int)(pair / (unsigned)a.TK), v);
+        tet_corners(a, (int)tet_of(a, pair), v);
         P4 g = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -2576,7 +2649,7 @@ hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, i
     return launch_lds(k_clip_plain<1, 1, 1>, grid, block, lds, st, a);
   }
   if (!a.site_counter || !a.units || !a.unit_count) return hipErrorInvalidValue;
-  if (a.rec_meta && (!a.rec_tris || !a.rec_count)) return hipErrorInvalidValue;
+  if (a.rec_meta && (!a.rec_tris || !a.rec_count || a.rec_chunk < 64)) return hipErrorInvalidValue;
   // the robust moments are never computed in the site-major kernel: the
   // polytopes it cannot hand to the volume pass go to the retry list
   if (moments == 1 && (!a.retry_list || !a.retry_count)) return hipErrorInvalidValue;
@@ -2620,7 +2693,8 @@ hipError_t tet_prep(const float4* tet_xyz, long long n, float4* out, hipStream_t
   return hipGetLastError();
 }
 
-hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* pair_count, hipStream_t st) {
+hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* out_ids, unsigned* pair_count,
+                      hipStream_t st) {
   if (a.n_sites <= 0) return hipSuccess;
   const int K = a.site_depth > 0 ? std::min(a.site_depth, a.K) : a.K;
   const int depth = std::min(a.cull_depth, K);
@@ -2631,7 +2705,13 @@ hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* pair_coun
 #endif
   const unsigned blocks =
       (unsigned)(kXcds * std::max(1, std::min((a.n_sites + kXcds - 1) / kXcds, VD_CULL_BLOCKS / kXcds)));
-  hipLaunchKernelGGL(k_cull_site, dim3(blocks), dim3(64), 32 * (size_t)depth, st, a, depth, pair_ids, pair_count);
+  const size_t lds = 20 * (size_t)depth + 4 * (27 + 1);
+  if (out_ids != pair_ids)
+    hipLaunchKernelGGL(k_cull_site<4>, dim3(blocks), dim3(256), lds + 4 * 4 * kCullQueue, st, a, depth, pair_ids,
+                       out_ids, pair_count);
+  else
+    hipLaunchKernelGGL(k_cull_site<1>, dim3(blocks), dim3(64), lds + 4 * kCullQueue, st, a, depth, pair_ids, out_ids,
+                       pair_count);
   return hipGetLastError();
 }
 
@@ -2711,7 +2791,7 @@ hipError_t cells_launch(const ClipArgs& a0, const CellStore& cs, int moments, in
     ac.cell_status = cs.status;
     ac.cell_nv = cs.nv;
     ac.cell_nt = cs.nt;
-    if ((e = cull_sites(ac, pair_ids, cull_count, st)) != hipSuccess) return e;
+    if ((e = cull_sites(ac, pair_ids, pair_ids, cull_count, st)) != hipSuccess) return e;
     a.pair_count = cull_count;
   }
   lds = cells_clip_lds(a.pcap, a.tcap);

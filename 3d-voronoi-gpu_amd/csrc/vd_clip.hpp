@@ -18,12 +18,14 @@ struct ClipArgs {
                              // loads them
   const int32_t* tet_knn;    // n_tets x TK candidate sites
   int TK;
+  unsigned tk_mul, tk_shift;   // division by TK (set_tk)
   long long n_pairs;         // n_tets * TK
   int n_sites;
   const unsigned* pair_start;  // site-major form: n_sites + 1
   const unsigned* pair_ids;  // site-major form: n_pairs pair indices grouped by site
   const unsigned* pair_count;  // site-major and cell forms, optional: only the first pair_count[s]
                                // pairs of site s's range are clipped (cull_sites' survivors)
+  float max_coord;             // cull_sites: the mesh's largest |coordinate|
   const int* cell_status;      // cell form, optional: cull_sites keeps every pair of a site
                                // whose cell was not built (its pairs take the cell's status),
   const int* cell_nv;          // or whose cell's plane / triangle counts could overflow the
@@ -54,6 +56,7 @@ struct ClipArgs {
   uint32_t* rec_tris;
   unsigned* rec_count;
   unsigned rec_cap;
+  unsigned rec_chunk;        // record slots a wave reserves at a time, per size class (64 and up)
   const unsigned* pair_list; // tet-major form: optional list of pairs to process
   const unsigned* pair_list_count;
   unsigned* srnr_list;       // optional: pairs ending security_radius_not_reached are listed
@@ -75,6 +78,16 @@ struct ClipArgs {
 // whatever its pairs were, with one set).
 constexpr int kHistStripes = 64, kHistStride = 16;
 constexpr int kHistWords = kHistStripes * kHistStride;
+
+// a.TK and the constants of a division by it.
+inline void set_tk(ClipArgs& a, int TK) {
+  a.TK = TK;
+  int l = 0;
+  while ((1ll << l) < TK) ++l;
+  const bool pow2 = TK < 1 || (1ll << l) == TK;
+  a.tk_mul = pow2 ? 0u : (unsigned)((((1ull << l) - (unsigned)TK) << 32) / (unsigned)TK + 1ull);
+  a.tk_shift = (unsigned)(pow2 ? l : l - 1);
+}
 
 // Cells of kernel B, kept for kernel C: per site its status, plane and
 // triangle counts, squared radius of its farthest vertex, planes [pcap] and
@@ -140,10 +153,12 @@ inline int exact_cull_depth(int depth, int pcap, int tcap) {
 
 // The site-major form's emptiness test as a pass of its own over the pairs
 // grouped by site (a.pair_start, pair_ids), with a.cull_depth bisectors (at
-// most 256; at most exact_cull_depth of the configured caps): the survivors of site s are moved, in order, to the front of its
-// range and their number written to pair_count[s]; a culled pair counts as
-// no_intersection (a.status_hist, a.pair_status, a.pair_vals).
-hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* pair_count, hipStream_t st);
+// most 256; at most exact_cull_depth of the configured caps): the survivors of
+// site s go to the front of its range in out_ids and their number to
+// pair_count[s]; a culled pair counts as no_intersection (a.status_hist,
+// a.pair_status, a.pair_vals).  out_ids: pair_ids itself (one wave per site),
+// or another buffer of its size (four, for small problems).
+hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* out_ids, unsigned* pair_count, hipStream_t st);
 // The work units of the site-major clipping: every site's pairs (the first
 // pair_count[s] of its range when given, else all) cut into runs of at most
 // unit_pairs, each (site, first pair position, number of pairs, 0), in the

@@ -71,6 +71,15 @@ constexpr int kFreshSiteDepth = 64;
 // 48,000 0.60 / 0.69, 82,944 (386k pieces) 0.80 / 0.77, 146,334 1.25 / 1.14.
 constexpr double kWidePieces = 256e3;
 constexpr int kWideDepth = 96, kWideTcap = 32;
+// Below this many sites the clipping's work units and the records that a wave
+// reserves at a time are smaller.
+constexpr int kSplitSites = 8192;
+// Up to this many sites the emptiness pass takes each with four waves (ten
+// iterations at 1,296 tets / 131 sites 3.05 ms against 3.16 with one, at 48,000
+// / 2,000 3.75 against 3.79 for six; at 82,944 / 8,294 7.24 against 7.12).
+constexpr int kFourWaveSites = 2048;
+// More waves than the GPU holds of the clipping kernel (9 per CU at most).
+constexpr long long kClipWaves = 2560;
 // kNN steps after the caller sets sites that do without the previous rows'
 // bounds (see vd_knn_step)
 constexpr int kHintAfter = 2;
@@ -186,6 +195,7 @@ struct vd_ctx {
   // site-major pairs
   DevBuf<int> p_count, p_cursor;
   DevBuf<unsigned> p_start, p_ids;
+  DevBuf<unsigned> p_ids2;  // survivors of the emptiness test by site (small problems)
   DevBuf<uint4> units;      // work units of the clipping
   DevBuf<unsigned> p_surv;  // survivors of the emptiness test per site
   // accumulators
@@ -468,7 +478,7 @@ void vd_ctx_destroy(vd_ctx* ctx) {
   ctx->g_cell_of.release(); ctx->g_sorted_ids.release(); ctx->g_sorted_pts.release();
   ctx->g_scan_tmp.release(); ctx->p_scan_tmp.release();
   ctx->site_knn.release(); ctx->tet_knn.release();
-  ctx->p_count.release(); ctx->p_start.release(); ctx->p_cursor.release(); ctx->p_ids.release(); ctx->p_surv.release(); ctx->units.release();
+  ctx->p_count.release(); ctx->p_start.release(); ctx->p_cursor.release(); ctx->p_ids.release(); ctx->p_ids2.release(); ctx->p_surv.release(); ctx->units.release();
   ctx->acc_f32.release(); ctx->acc_fix.release(); ctx->moments.release();
   ctx->pair_status.release(); ctx->pair_vals.release(); ctx->hist.release();
   ctx->retry_list.release(); ctx->retry_list2.release();
@@ -797,7 +807,9 @@ int vd_clip_step(vd_ctx* ctx) {
   a.tet_xyz = ctx->tet_xyz.p;
   a.tet_prep = ctx->tet_prep.p;
   a.tet_knn = ctx->tet_knn.p;
-  a.TK = ctx->TK;
+  vd::set_tk(a, ctx->TK);
+  for (int x = 0; x < 3; ++x)
+    a.max_coord = std::max({a.max_coord, std::fabs(ctx->mesh_lo[x]), std::fabs(ctx->mesh_hi[x])});
   a.n_pairs = n_pairs;
   a.n_sites = n;
   a.pcap = c.pcap;
@@ -872,8 +884,14 @@ int vd_clip_step(vd_ctx* ctx) {
     a.cull_depth = vd::exact_cull_depth(c.cull_depth, c.pcap, c.tcap);
     if (std::min(a.cull_depth, a.site_depth) > 0) {
       // the emptiness test as a pass of its own; the clipping takes the survivors
+      unsigned* out = ctx->p_ids.p;
+      if (n <= kFourWaveSites) {
+        VD_HIP(ctx->p_ids2.ensure(std::max(n_pairs, 1LL)), "alloc pairs");
+        out = ctx->p_ids2.p;
+      }
       VD_HIP(ctx->p_surv.ensure(n), "alloc pairs");
-      VD_HIP(vd::cull_sites(a, ctx->p_ids.p, ctx->p_surv.p, ctx->stream), "cull");
+      VD_HIP(vd::cull_sites(a, ctx->p_ids.p, out, ctx->p_surv.p, ctx->stream), "cull");
+      a.pair_ids = out;
       a.pair_count = ctx->p_surv.p;
       a.cull_depth = 0;
     }
@@ -883,19 +901,22 @@ int vd_clip_step(vd_ctx* ctx) {
     // iterations), 820k torus tets (2), 48,000 tets / 2,000 sites (1): 32 pairs
     // 93.9, 47.7, 1.12; 64 79.3, 44.9, 1.04; 128 75.3, 44.2, 1.06; 256 75.2,
     // 44.5, 1.16; 1,024 75.3, 45.7, 1.24.
-    const int unit = n < 8192 ? 64 : 128;
+    const int unit = n < kSplitSites ? 64 : 128;
     VD_HIP(ctx->units.ensure((size_t)vd::max_site_units(n_pairs, n, unit)), "alloc units");
     VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
     a.units = ctx->units.p;
     a.unit_count = ctx->counter(vd_ctx::kUnitCount);
     if (c.site_records >= 0) {
-      // automatic: the estimate, plus the slots the waves reserve ahead
+      // automatic: the estimate, plus the slots that the waves reserve ahead (a
+      // chunk of each size class per wave; smaller chunks where every wave has
+      // few pairs)
+      a.rec_chunk = n < kSplitSites ? 64 : 128;
       const long long more =
           (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
-      const long long want = c.site_records > 0
-                                 ? c.site_records
-                                 : n_pairs / 10 + std::max(0LL, std::min(more, ctx->more_records)) + 262144;
-      const unsigned cap = (unsigned)std::max(1LL, std::min({want, n_pairs, (long long)UINT32_MAX}));
+      const long long ahead = 2LL * a.rec_chunk * std::min(kClipWaves, vd::max_site_units(n_pairs, n, unit));
+      const long long want = c.site_records > 0 ? std::min(c.site_records + 0LL, n_pairs)
+                                                : n_pairs / 10 + std::max(0LL, std::min(more, ctx->more_records)) + ahead;
+      const unsigned cap = (unsigned)std::max(1LL, std::min(want, (long long)UINT32_MAX));
       VD_HIP(ctx->rec_meta.ensure(cap), "alloc records");
       VD_HIP(ctx->rec_tris.ensure((size_t)cap * vd::rec_stride(fast_tcap)), "alloc records");
       a.rec_meta = ctx->rec_meta.p;

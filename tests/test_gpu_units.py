@@ -61,3 +61,24 @@ def test_records_at_few_candidates(vdn, O, n, ns, tk):
             e.knn_step()
             e.clip_step()
             np.testing.assert_array_equal(e.moments(), r["site_vals"])
+
+
+@pytest.mark.parametrize("n,ns,tk,depth", [(5, 30, 30, 1), (9, 2048, 40, 16), (9, 2049, 40, 16), (8, 90, 64, 2),
+                                           (12, 400, 33, 90)])
+def test_emptiness_pass_bit_exact(vdn, O, n, ns, tk, depth):
+    """The emptiness pass with one and four waves per site, at few and many
+    bisectors, at candidate counts that are and are not powers of two."""
+    verts, tets, sites = problem("cube", n, ns)
+    sk, tkn = oracle_knn("cube", n, ns, 90, tk)
+    r = O.clip_tets(sites, sk, verts, tets, tkn, geom="f32", pair_acc="f64", site_mode=O.SITE_FIXED, moments="robust")
+    with vdn.Engine(tet_k=tk, accum="f64", moments="robust", record_pairs=1, cull_depth=depth) as e:
+        e.set_mesh(verts, tets)
+        e.set_sites(sites)
+        e.knn_step()
+        e.clip_step()
+        st, vals = e.pairs()
+        np.testing.assert_array_equal(st.astype(np.int32), r["pair_status"])
+        np.testing.assert_array_equal(vals, r["pair_vals"])
+        np.testing.assert_array_equal(e.moments(), r["site_vals"])
+        hist = e.status_hist()
+        assert [hist[k] for k in vdn.STATUS_NAMES] == np.bincount(r["pair_status"], minlength=7).tolist()
