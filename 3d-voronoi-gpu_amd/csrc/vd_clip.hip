@@ -2169,6 +2169,201 @@ __global__ __launch_bounds__(64) void k_cells(ClipArgs a, CellStore cs, int pstr
   }
 }
 
+// Kernel B with a wavefront per site: lane t holds vertex t of the cell (plane
+// triple, squared distance to the seed, the minors of its planes), lane p the
+// boundary link of plane p, LDS the planes; at most 64 of either.  A bisector
+// is tested against every vertex at once (a 4-term determinant per lane), the
+// removal and the boundary walk are uniform over the wave and run on lane reads
+// and writes, and the fan's new vertices are computed one per lane.  Triangles
+// are removed, walked and added in the order of Cell::clip, so a cell that
+// succeeds or misses the security radius is the same cell bit for bit; every
+// other outcome (a cap, a failed walk, an empty cell, a bad neighbour id) is
+// listed for k_cells.
+//
+// One lane per site (k_cells) left the GPU with n / 64 waves, each as slow as
+// its slowest lane's chain of dependent LDS reads: at 384,000 tets / 38,400
+// sites 2.11 and 1.09 ms (iterations 1 and 2), now 0.61 and 0.51; at 3,001 sites
+// 0.46-1.09 ms, now 0.07-0.11.
+constexpr int kCellWaves = 4;
+constexpr int kCellMax = 64;        // planes and vertices
+constexpr int kCellWalkMax = 4096;  // steps of a boundary walk (k_cells has the reference's guard)
+
+__device__ __forceinline__ int rdlane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ float rdlane(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
+}
+__device__ __forceinline__ int wrlane(int v, int x, int l) { return (int)(threadIdx.x & 63) == l ? x : v; }
+__device__ __forceinline__ int gather(int v, int l) { return __builtin_amdgcn_ds_bpermute(l << 2, v); }
+__device__ __forceinline__ float gather(float v, int l) {
+  return __int_as_float(__builtin_amdgcn_ds_bpermute(l << 2, __float_as_int(v)));
+}
+// Largest of the lanes' values and 0 (NaN ignored), in every lane.
+__device__ __forceinline__ float wave_max0(float x) {
+  auto from = [](float v, auto ctrl, auto rows) {
+    return __int_as_float(
+        __builtin_amdgcn_update_dpp(0, __float_as_int(v), decltype(ctrl)::value, decltype(rows)::value, 0xF, false));
+  };
+  x = fmaxf(x, 0.f);
+  x = fmaxf(x, from(x, std::integral_constant<int, 0x111>(), std::integral_constant<int, 0xF>()));  // row_shr:1
+  x = fmaxf(x, from(x, std::integral_constant<int, 0x112>(), std::integral_constant<int, 0xF>()));  // row_shr:2
+  x = fmaxf(x, from(x, std::integral_constant<int, 0x114>(), std::integral_constant<int, 0xF>()));  // row_shr:4
+  x = fmaxf(x, from(x, std::integral_constant<int, 0x118>(), std::integral_constant<int, 0xF>()));  // row_shr:8
+  x = fmaxf(x, from(x, std::integral_constant<int, 0x142>(), std::integral_constant<int, 0xA>()));  // row_bcast:15
+  x = fmaxf(x, from(x, std::integral_constant<int, 0x143>(), std::integral_constant<int, 0xC>()));  // row_bcast:31
+  return rdlane(x, 63);
+}
+
+// pcap, tcap: the launch's caps (at most kCellMax); the rest as k_cells.
+__global__ __launch_bounds__(64 * kCellWaves) void k_cells_wave(ClipArgs a, CellStore cs, int pcap, int tcap,
+                                                                int pstride, int tstride, unsigned* redo_out) {
+  __shared__ float4 planes_all[kCellWaves][kCellMax];
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  float4* pl = planes_all[wv];
+  const int s = __builtin_amdgcn_readfirstlane((int)blockIdx.x * kCellWaves + wv);
+  if (s >= a.n_sites) return;
+  const P4 sp = site_at(a, s);
+  const int32_t* nbr = a.site_knn + (size_t)s * a.K;
+  // box start (Cell::init_box)
+  const float lo = -0.1f, hi = 1000.f + 0.1f;
+  if (lane < 6) {
+    const float sg = (lane & 1) ? -1.f : 1.f, w = (lane & 1) ? hi : -lo;
+    pl[lane] = make_float4(lane < 2 ? sg : 0.f, lane >= 2 && lane < 4 ? sg : 0.f, lane >= 4 ? sg : 0.f, w);
+  }
+  int tri = 0;
+  {
+    const int box[8] = {(int)pack3(2, 5, 0), (int)pack3(5, 3, 0), (int)pack3(1, 5, 2), (int)pack3(5, 1, 3),
+                        (int)pack3(4, 2, 0), (int)pack3(4, 0, 3), (int)pack3(2, 4, 1), (int)pack3(4, 3, 1)};
+#pragma unroll
+    for (int t = 0; t < 8; ++t) tri = lane == t ? box[t] : tri;
+  }
+  wave_fence();
+  int nt = 8, nv = 6;
+  float d2 = 0.f, vmax = 0.f;
+  Minors mn = {0.f, 0.f, 0.f, 0.f};
+  // the vertices of lanes [first_lane, nt): distance and minors from their planes
+  auto make_vertices = [&](int first_lane) {
+    if (lane >= first_lane && lane < nt) {
+      const P4 p1 = ld4(pl, tri_a(tri)), p2 = ld4(pl, tri_b(tri)), p3 = ld4(pl, tri_c(tri));
+      const P4 d = sub3(vertex3(p1, p2, p3), sp);
+      d2 = dot3(d, d);
+      mn = vertex_minors(p1, p2, p3);
+    }
+    vmax = wave_max0(lane < nt ? d2 : 0.f);
+  };
+  make_vertices(0);
+  bool failed = false, stopped = false;
+  float ex = 0.f, ey = 0.f, ez = 0.f, ew = 0.f, ed = 0.f;
+  unsigned long long bad = 0;
+  for (int v = 0; v < a.K && !failed && !stopped; ++v) {
+    if ((v & 63) == 0) {
+      // the next 64 bisectors, one per lane
+      const int j = v + lane;
+      const int z = j < a.K ? nbr[j] : 0;
+      const bool ok = (unsigned)z < (unsigned)a.n_sites;
+      const P4 zp = site_at(a, ok ? z : 0);
+      const P4 e = bisector(sp, zp), d = sub3(zp, sp);
+      ex = e.x; ey = e.y; ez = e.z; ew = e.w;
+      ed = dot3(d, d);
+      bad = __ballot(!ok);
+    }
+    const int l = v & 63;
+    if ((bad >> l) & 1ull || nv >= pcap) {
+      failed = true;
+      break;
+    }
+    const P4 e = {rdlane(ex, l), rdlane(ey, l), rdlane(ez, l), rdlane(ew, l)};
+    const float d2z = rdlane(ed, l);
+    unsigned long long conf = __ballot(lane < nt && conflict_det(mn, e) > 0.f);
+    if (conf != 0) {
+      const int pid = nv++;
+      if (lane == 0) pl[pid] = make_float4(e.x, e.y, e.z, e.w);
+      // removal: ascending slot, a conflicting slot takes the last live one
+      // (Cell::cut_remove), replayed on the slots' numbers
+      int perm = lane, n = nt, nr = 0;
+      while (conf) {
+        const int i = __builtin_ctzll(conf);
+        --n;
+        ++nr;
+        const unsigned long long bi = 1ull << i, bn = 1ull << n;
+        const int pi = rdlane(perm, i), pn = rdlane(perm, n);
+        perm = wrlane(wrlane(perm, pn, i), pi, n);
+        conf = (conf & ~(bi | bn)) | (i != n && (conf & bn) ? bi : 0ull);
+      }
+      if (n == 0) {
+        failed = true;
+        break;
+      }
+      tri = gather(tri, perm);
+      d2 = gather(d2, perm);
+      mn.m123 = gather(mn.m123, perm);
+      mn.m124 = gather(mn.m124, perm);
+      mn.m134 = gather(mn.m134, perm);
+      mn.m234 = gather(mn.m234, perm);
+      // boundary walk (Cell::walk_steps)
+      int nx = kNoPlane, first = kNoPlane, cur = n, guard = 0;
+      while (nr > 0) {
+        if (guard++ > kCellWalkMax) {
+          failed = true;
+          break;
+        }
+        const uint32_t t = (uint32_t)rdlane(tri, cur);
+        const int e0 = tri_a(t), e1 = tri_b(t), e2 = tri_c(t);
+        const int n0 = rdlane(nx, e0), n1 = rdlane(nx, e1), n2 = rdlane(nx, e2);
+        const bool on0 = n0 != kNoPlane, on1 = n1 != kNoPlane, on2 = n2 != kNoPlane;
+        const bool op0 = n1 == e0, op1 = n2 == e1, op2 = n0 == e2;
+        const bool none = !op0 && !op1 && !op2;
+        if ((!op0 && !op1 && on1) || (!op1 && !op2 && on2) || (!op2 && !op0 && on0) || (none && first != kNoPlane)) {
+          ++cur;
+          if (cur == n + nr) cur = n;
+          continue;
+        }
+        if (none) first = e0;
+        if (op0 && op1 && first == e1) first = n1;
+        if (op1 && op2 && first == e2) first = n2;
+        if (op2 && op0 && first == e0) first = n0;
+        nx = wrlane(nx, op2 && op0 ? kNoPlane : (op0 ? n0 : e1), e0);
+        nx = wrlane(nx, op0 && op1 ? kNoPlane : (op1 ? n1 : e2), e1);
+        nx = wrlane(nx, op1 && op2 ? kNoPlane : (op2 ? n2 : e0), e2);
+        tri = wrlane(tri, rdlane(tri, n + nr - 1), cur);
+        cur = n;
+        --nr;
+      }
+      if (failed) break;
+      // fan of new vertices around plane pid (Cell::fan_steps)
+      nt = n;
+      if (first != kNoPlane) {
+        int c = first;
+        do {
+          const int nn = rdlane(nx, c);
+          if (nn == kNoPlane || nt + 1 >= tcap) {
+            failed = true;
+            break;
+          }
+          tri = wrlane(tri, (int)pack3(pid, c, nn), nt);
+          ++nt;
+          c = nn;
+        } while (c != first);
+        if (failed) break;
+      }
+      wave_fence();  // the new plane
+      make_vertices(n);
+    }
+    stopped = d2z > 4.f * vmax;
+  }
+  if (failed) {
+    if (lane == 0) redo_out[1 + atomicAdd(redo_out, 1u)] = (unsigned)s;  // each site once: below n_sites entries
+    return;
+  }
+  if (lane == 0) {
+    cs.status[s] = stopped ? kSuccess : kSecurityRadiusNotReached;
+    cs.nv[s] = nv;
+    cs.nt[s] = nt;
+    cs.r2[s] = vmax;
+  }
+  if (lane < nv) cs.planes[(size_t)s * pstride + lane] = pl[lane];
+  if (lane < nt) cs.tris[(size_t)s * tstride + lane] = (uint32_t)tri;
+}
+
 // pstride / tstride: the cell store's planes and triangles per site; part 0
 // takes the sites whose cell has fewer than split - 8 triangles and at most
 // psplit - 4 planes (and the cells that were not built), part 1 the other
@@ -2765,13 +2960,21 @@ hipError_t cells_launch(const ClipArgs& a0, const CellStore& cs, int moments, in
   hipError_t e = hipFuncSetAttribute((const void*)k_cells<0>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (e != hipSuccess) return e;
   ClipArgs ab = a0;
-  ab.pcap = std::min(a0.pcap, fast_pcap > 0 ? fast_pcap : kCellsFastPcap);
-  ab.tcap = std::min(a0.tcap, fast_tcap > 0 ? fast_tcap : kCellsFastTcap);
-  const bool redo = cs.redo && (ab.pcap < a0.pcap || ab.tcap < a0.tcap);
+  const bool wave = a0.filter == 0 && cs.redo;
+  ab.pcap = std::min(a0.pcap, fast_pcap > 0 ? fast_pcap : (wave ? kCellMax : kCellsFastPcap));
+  ab.tcap = std::min(a0.tcap, fast_tcap > 0 ? fast_tcap : (wave ? kCellMax : kCellsFastTcap));
+  const bool redo = wave || (cs.redo && (ab.pcap < a0.pcap || ab.tcap < a0.tcap));
   if (!redo) ab = a0;
   if (redo && (e = fill_u32(cs.redo, 1, 0u, st)) != hipSuccess) return e;
-  hipLaunchKernelGGL(k_cells<0>, dim3((unsigned)((a0.n_sites + 63) / 64)), dim3(64), cells_lds(ab.pcap, ab.tcap), st, ab,
-                     cs, a0.pcap, a0.tcap, redo ? cs.redo : nullptr, (const unsigned*)nullptr);
+  if (wave) {
+    hipLaunchKernelGGL(k_cells_wave, dim3((unsigned)((a0.n_sites + kCellWaves - 1) / kCellWaves)),
+                       dim3(64 * kCellWaves), 0, st, a0, cs, std::min(ab.pcap, kCellMax), std::min(ab.tcap, kCellMax),
+                       a0.pcap, a0.tcap, cs.redo);
+  } else {
+    // the arithmetic filter's tests have side effects: one lane per site
+    hipLaunchKernelGGL(k_cells<0>, dim3((unsigned)((a0.n_sites + 63) / 64)), dim3(64), cells_lds(ab.pcap, ab.tcap), st,
+                       ab, cs, a0.pcap, a0.tcap, redo ? cs.redo : nullptr, (const unsigned*)nullptr);
+  }
   if ((e = hipGetLastError()) != hipSuccess) return e;
   if (redo) {
     // the listed sites at the configured caps (64 workgroups, looping over

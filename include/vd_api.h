@@ -107,10 +107,9 @@ typedef struct vd_config {
                          a small problem) */
   int knn_waves;      /* wavefronts per workgroup of the kNN queries: 2, 4 or 8; 0 = automatic
                          (4); results do not depend on it */
-  int cells_pcap;     /* cell form: plane cap of kernel B's first launch (8..pcap); cells that
-                         fail there are built again at pcap/tcap, so results do not depend on
-                         it; 0 = automatic (40: with cells_tcap 64, two waves per CU instead
-                         of one at 64/96) */
+  int cells_pcap;     /* cell form: plane cap of kernel B's first launch (8..pcap, at most 64
+                         with filter 0); cells that fail there are built again at pcap/tcap, so
+                         results do not depend on it; 0 = automatic (64; 40 with the filter) */
   int cells_tcap;     /* cell form: vertex cap of kernel B's first launch (8..tcap), likewise;
                          0 = automatic (64) */
 } vd_config;
