@@ -2384,7 +2384,11 @@ __global__ __launch_bounds__(64) void k_cells_clip(ClipArgs a, CellStore cs, int
   uint8_t* nx = (uint8_t*)(tr + (size_t)a.tcap * 64);       // [pcap][64]
   int* surv = (int*)(nx + (size_t)a.pcap * 64);             // [128] queued pairs
   uint8_t* sslot = (uint8_t*)(surv + 128);                  // [128] their slots
-  float4* fl = (float4*)(((uintptr_t)(sslot + 128) + 15) & ~(uintptr_t)15);  // [4][64]
+  // [4][64], from the base by an offset (rounded up as a pointer, the compiler
+  // no longer knows it for LDS and reads every plane by a flat load: two
+  // iterations at 384,000 tets / 38,400 sites 16.8 -> 16.2 ms)
+  const size_t fl_off = (size_t)(sslot + 128 - smem);
+  float4* fl = (float4*)(smem + ((fl_off + 15) & ~(size_t)15));
   Cell<PlaneStoreCell, TriPlain> c;
   c.ps.fl = fl;
   c.ps.lane = lane;
