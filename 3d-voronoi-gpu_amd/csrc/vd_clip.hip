@@ -689,21 +689,26 @@ struct Cell {
       vmax = m;
       return d2z > 4.f * m ? 1 : 0;
     }
-    int c = first;
-    int guard = 0;
     // the new vertex (pid, c, n): the plane of pid and of c are already in
     // registers (c is the previous vertex's n), one plane read per vertex
     const P4 pp = ps.get(pid);
     P4 pc = ps.get(first);
-    // one exit for the three failures (an open or runaway loop, the vertex
-    // cap), taken before anything is stored for the failing vertex
-    // (err: the failure status, or -1; kTriangleOverflow is 0)
+    // the loop ends without closing at the vertex cap, after more than pcap
+    // steps, or where it is open, before anything is stored for that vertex: one
+    // test and one exit a step (10 iterations at 1M tets / 100,000 sites 66.3
+    // -> 65.8 ms; with the next link read ahead 66.0, and with one reciprocal
+    // shared by a vertex's three quotients no faster)
+    const int most = min(pcap + 1, tcap - 1 - nt);
+    const int nt_end = nt + most;
+    const bool runaway = most == pcap + 1;
     int err = -1;
+    int c = first;
     do {
-      err = (c == kNoPlane || guard++ > pcap) ? kInconsistentBoundary : (nt + 1 >= tcap ? kTriangleOverflow : -1);
-      const int n = err >= 0 ? kNoPlane : nxt(c);
-      if (err < 0 && n == kNoPlane) err = kInconsistentBoundary;
-      if (err >= 0) break;
+      const int n = nxt(c);
+      if (nt >= nt_end || n == kNoPlane) {
+        err = nt < nt_end || runaway ? kInconsistentBoundary : kTriangleOverflow;
+        break;
+      }
       const P4 pn = ps.get(n);
       const float d = seed_d2(vertex3(pp, pc, pn));
       ts.put(nt, pack3(pid, c, n), d);
