@@ -447,15 +447,23 @@ int vd_ctx_create(vd_ctx** out, int device, const vd_config* cfg) {
     delete ctx;
     return VD_ERR_HIP;
   }
+  // No system-scope fence (a cache write-back of 2 to 6 us on the stream) at
+  // these events: nobody waits for them on the host, the fork and join events
+  // order kernels of one device, which release to the device as they end, and
+  // results are read after the stream's own synchronisation.  Five phase
+  // events and up to four forks and joins an iteration: 10 iterations at 1,296
+  // tets 2.93 -> 2.74 ms (2.80 with the phase events alone), at 10,368 tets
+  // 3.93 -> 3.78.
+  const unsigned order = hipEventDisableTiming | hipEventDisableSystemFence;
   if (hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming) != hipSuccess ||
-      hipEventCreateWithFlags(&ctx->join_ev, hipEventDisableTiming) != hipSuccess) {
+      hipEventCreateWithFlags(&ctx->fork_ev, order) != hipSuccess ||
+      hipEventCreateWithFlags(&ctx->join_ev, order) != hipSuccess) {
     fprintf(stderr, "vd_ctx_create: cannot create the kNN step's second stream on device %d\n", device);
     vd_ctx_destroy(ctx);
     return VD_ERR_HIP;
   }
   for (auto& row : ctx->ev)
-    for (auto& e : row) (void)hipEventCreate(&e);
+    for (auto& e : row) (void)hipEventCreateWithFlags(&e, hipEventDisableSystemFence);
   if (ensure_offsets(ctx) != VD_OK || ctx->hist.ensure(vd_ctx::kCounterWords / 2) != hipSuccess) {
     fprintf(stderr, "vd_ctx_create: %s\n", ctx->err.c_str());
     vd_ctx_destroy(ctx);
