@@ -1244,7 +1244,7 @@ hipError_t scan_excl(const int* in, const int* n_dev, int n_max, unsigned* out, 
   return scan_excl_t<unsigned>(in, n_dev, n_max, out, cursor, tmp, st);
 }
 
-std::vector<int4> knn_offset_table() {
+static std::vector<int4> make_offset_table() {
   std::vector<int4> t;
   const int R = kOffsetRadius;
   for (int z = -R; z <= R; ++z)
@@ -1259,6 +1259,10 @@ std::vector<int4> knn_offset_table() {
     const int cb = std::max(std::abs(b.x), std::max(std::abs(b.y), std::abs(b.z)));
     return ca < cb;
   });
+  return t;
+}
+const std::vector<int4>& knn_offset_table() {
+  static const std::vector<int4> t = make_offset_table();
   return t;
 }
 
