@@ -766,6 +766,23 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
   // q0 + j once it is known (-2 before; -1: that row gives none)
   const bool use_hint = a.hint_pts && a.out_pitch <= 0 && (a.mode == 0 || a.mode == 1);
   float run_hb = -2.f;
+  // Results by columns (pitched, one column per query) that wait to be written
+  // together: n_held queries from q_held on, in the space of the point list
+  // while there is none.  A row of such a result has the run's queries side by
+  // side, and one store then covers ten rows instead of 64.
+  const bool hold = a.out_pitch > 0 && (a.mode == 1 || a.mode == 2) && run > 1;
+  int* held = (int*)uni;  // [n_held][a.k + 1]
+  static_assert(kQueryRun * (256 + 1) * sizeof(int) <= kUnionCap * sizeof(float4), "held results");
+  int n_held = 0, q_held = q0;
+  auto write_held = [&]() {
+    if (n_held == 0) return;
+    wave_sync();
+    const int rows = 64 / n_held, j0 = lane / n_held, i = lane - j0 * n_held;
+    if (j0 < rows)
+      for (int j = j0; j < a.k; j += rows) a.out[(long long)j * a.out_pitch + q_held + i] = held[i * (a.k + 1) + j];
+    wave_sync();
+    n_held = 0;
+  };
   // The run's point list: every point of the instance within sqrt(R2) of c,
   // with its id in w; returns their number, or -1 when they do not fit in
   // kUnionCap or the offset table does not reach that far (beyond it the
@@ -1030,12 +1047,18 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
     const int j = s * 64 + lane;
     if (j < a.k) {
       const int32_t id = L.s[s] == kNoKey ? -1 : (int32_t)(uint32_t)L.s[s];
-      if (a.out_pitch > 0)
+      if (hold && n_uni < 0)
+        held[(q - q_held) * (a.k + 1) + j] = id;
+      else if (a.out_pitch > 0)
         a.out[(long long)j * a.out_pitch + out_row] = id;
       else
         a.out[(long long)out_row * a.k + j] = id;
     }
   }
+  if (hold && n_uni < 0)
+    ++n_held;
+  else
+    q_held = q + 1;
   const uint64_t kth = topk_kth<M>(L, a.k);
   prev_r = kth == kNoKey ? -1.f : sqrtf(key_d2(kth));
   prev_qp = qp;
@@ -1084,16 +1107,26 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
       // rounding margins of the FP32 distances on either side
       const float R = rj_need * (1.f + 1e-4f) + 1e-3f * g.h;
       const float R2 = R * R;
-      const int n = gather(c, R2, g, cbase);
-      if (n >= 0) {
-        n_uni = n;
-        uni_inst = inst;
-        r0 = prev_r;
-        q0p = qp;
+      // A ball of radius R as densely filled as the first query's holds
+      // k (R / r0)^3 points; a gather of far more than the list takes (queries
+      // in no spatial order) would fail after reading most of them: 100,000
+      // points, 1M random queries 2.45 -> 2.24 ms, and 2.13 with the results held as above.
+      const float rel = R / prev_r;
+      if (!((float)a.k * rel * rel * rel > 2.f * (float)kUnionCap && prev_r > 0.f)) {
+        write_held();  // the list takes their space
+        q_held = q + 1;
+        const int n = gather(c, R2, g, cbase);
+        if (n >= 0) {
+          n_uni = n;
+          uni_inst = inst;
+          r0 = prev_r;
+          q0p = qp;
+        }
       }
     }
   }
   }  // query loop
+  write_held();
 }
 
 }  // namespace
