@@ -700,10 +700,20 @@ constexpr int kQueryRun = VD_KNN_RUN, kQueryFill = VD_KNN_FILL;
 // centre c of the run.  Those queries scan the list instead of walking the
 // grid, with the same keys and the same bounds, so their results are the
 // same; a run whose list would not fit walks as before.
-#ifndef VD_KNN_UNION_CAP
-#define VD_KNN_UNION_CAP 512
-#endif
-constexpr int kUnionCap = VD_KNN_UNION_CAP;
+//
+// What bounds the kernel is the issue of vector instructions, with 4 waves per
+// SIMD not quite: at 5 the list is held to the LDS of a fifth of a CU (lists of
+// tet queries, M = 1, take some 110 points, of site queries, M = 2, some 350)
+// and the registers to a fifth of a SIMD's.  kNN phase at 1M tets / 100,000
+// sites 1.55 -> 1.42 ms, 100,000 points and 1M random queries 2.14 -> 1.99 (M =
+// 1 with 192 or 320 points 1.44, M = 2 with 320 points 1.43, with 448 and 4
+// waves 1.49; 6 waves spill: 1.98).  Past k = 128 the list is longer, at the 3
+// waves that the registers allow.
+template <int M>
+struct QueryShape {
+  static constexpr int kUnionCap = M == 1 ? 256 : M == 2 ? 384 : 512;
+  static constexpr int kWavesPerSimd = M <= 2 ? 5 : 3;
+};
 
 // At most this many keys staged after the last merge are inserted one at a
 // time instead of sorted and merged.
@@ -742,7 +752,8 @@ __device__ __forceinline__ void query_point(const QueryArgs& a, int q, float4& q
 }
 
 template <int M, int kQueryWaves>
-__global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
+__global__ __launch_bounds__(64 * kQueryWaves, QueryShape<M>::kWavesPerSimd) void k_knn_query(QueryArgs a) {
+  constexpr int kUnionCap = QueryShape<M>::kUnionCap;
   __shared__ uint64_t stage_all[kQueryWaves][128];
   __shared__ int mark_all[kQueryWaves][64];  // batch_owner's marks
   __shared__ float4 uni_all[kQueryWaves][kUnionCap];  // (x, y, z, id bits)
@@ -772,7 +783,7 @@ __global__ __launch_bounds__(64 * kQueryWaves) void k_knn_query(QueryArgs a) {
   // side, and one store then covers ten rows instead of 64.
   const bool hold = a.out_pitch > 0 && (a.mode == 1 || a.mode == 2) && run > 1;
   int* held = (int*)uni;  // [n_held][a.k + 1]
-  static_assert(kQueryRun * (256 + 1) * sizeof(int) <= kUnionCap * sizeof(float4), "held results");
+  static_assert(kQueryRun * (64 * M + 1) * sizeof(int) <= kUnionCap * sizeof(float4), "held results");
   int n_held = 0, q_held = q0;
   auto write_held = [&]() {
     if (n_held == 0) return;
