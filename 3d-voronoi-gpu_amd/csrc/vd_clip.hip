@@ -2615,8 +2615,14 @@ __global__ __launch_bounds__(64) void k_cells_clip(ClipArgs a, CellStore cs, int
 // the global counter once; the scatter pass reserves one range per (block,
 // site) the same way.  Sites that do not fit the table go through global
 // atomics directly.  The order inside a site's list is unspecified.
+//
+// Pairs per block of the count: 8,192 fill the table of 2,048 with the sites of
+// an irregular mesh (probing grows long), 4,096 reserve more often.  Counting and
+// scattering at 820k torus tets / 200,000 sites, tet_k 96: 8,192 0.97 ms, 6,144
+// 0.65, 4,096 0.67, 2,048 0.76; 1M tets / 100,000 sites, tet_k 64: 0.53, 0.52,
+// 0.52, 0.56 (16,384: 6.96 and 0.60; a table of 1,024: 3.69 and 0.54).
 #ifndef VD_GROUP_PAIRS
-#define VD_GROUP_PAIRS 8192
+#define VD_GROUP_PAIRS 6144
 #endif
 #ifndef VD_GROUP_HASH_BITS
 #define VD_GROUP_HASH_BITS 11
