@@ -2119,18 +2119,21 @@ __global__ __launch_bounds__(kMomentsBlock) void k_site_moments(ClipArgs a) {
 //
 // Kernel B (voronoi.cu:540-575, 648-660): every site's Voronoi cell, the box
 // [-0.1, 1000.1]^3 clipped by the bisectors of the site's neighbours with the
-// security-radius exit; one lane per site; the cell (planes, triangles) is
-// stored for kernel C with the squared radius of its farthest vertex.
+// security-radius exit; a wave per site (k_cells_wave), or one lane per site
+// (k_cells) for the cells that it gives up and with the arithmetic filter; the
+// cell (planes, triangles) is stored for kernel C with the squared radius of its farthest vertex.
 // Kernel C (voronoi.cu:620-645, 703-726): for every (tet, site) pair, the
 // stored cell clipped by the tet's four face planes, then volume and moments
 // as in kernel A.  Site-major: a wavefront takes its sites one after another,
 // loads each site's cell into one of two LDS slots and queues the site's
 // pairs; every 64 queued pairs (of one or two sites) are clipped together.
 
-// Kernel B's launches: every site at caps of at most kCellsFastPcap planes
-// and kCellsFastTcap vertices (76 KB of LDS per wave, two waves per CU
-// instead of one at 64/96), then the sites whose cell failed there (the
-// redo list, about 4 in 100k seeded cells at 40/64) at the configured caps.
+// Kernel B's launches: every site at smaller caps than the configured ones
+// (k_cells_wave: a lane per plane and triangle, at most 64; k_cells, with the
+// filter: kCellsFastPcap planes and kCellsFastTcap vertices, 76 KB of LDS per
+// wave, two waves per CU instead of one at 64/96), then the sites whose cell
+// failed there (the redo list, about 4 in 100k seeded cells at 40/64) at the
+// configured caps.
 // A cell that succeeds at the smaller caps ran the same steps the configured
 // caps run (a cap only ends a build), so it is the same cell; every other
 // outcome is built again, since a runaway boundary walk's guard depends on
