@@ -338,10 +338,17 @@ struct Cell {
       bhi[1] = fmaxf(fmaxf(X[0].y, X[1].y), fmaxf(X[2].y, X[3].y)) - s.y;
       bhi[2] = fmaxf(fmaxf(X[0].z, X[1].z), fmaxf(X[2].z, X[3].z)) - s.z;
     } else {
-      ts.put(0, pack3(1, 3, 2), 0.f);
-      ts.put(1, pack3(0, 1, 2), 0.f);
-      ts.put(2, pack3(0, 3, 1), 0.f);
-      ts.put(3, pack3(0, 2, 3), 0.f);
+      P4 X[4];
+      float d2[4] = {0.f, 0.f, 0.f, 0.f};
+      if constexpr (TS::kHasD2) {
+        corners_of(rec[4], rec[5], rec[6], X);
+#pragma unroll
+        for (int k = 0; k < 4; ++k) d2[k] = seed_d2(X[k]);
+      }
+      ts.put(0, pack3(1, 3, 2), d2[0]);
+      ts.put(1, pack3(0, 1, 2), d2[1]);
+      ts.put(2, pack3(0, 3, 1), d2[2]);
+      ts.put(3, pack3(0, 2, 3), d2[3]);
       vmax = 0.f;
     }
   }
@@ -1166,14 +1173,16 @@ __global__ __launch_bounds__(256) void k_tet_prep(const float4* tet_xyz, long lo
 
 // ------------------------------------------------------------ tet-major ----
 
-// CACHED: vertices stored with their distance to the seed (at most 32 per
+// CACHED 1: vertices stored with their distance to the seed (at most 32 per
 // polytope), as in the site-major form; used to re-clip the pairs that
-// overflow the site-major launch's smaller vertex cap.
+// overflow the site-major launch's smaller vertex cap.  CACHED 2: the
+// distances only, for the security test, at any vertex cap.
 template <int MF, int ACC, int CACHED>
 __global__ __launch_bounds__(64) void k_clip_plain(ClipArgs a) {
   extern __shared__ __align__(16) uint8_t smem[];
   const int lane = threadIdx.x;
-  using TS = typename std::conditional<CACHED != 0, TriCached, TriPlain>::type;
+  using TS = typename std::conditional<CACHED == 1, TriCached,
+                                       typename std::conditional<CACHED == 2, TriPlainD2, TriPlain>::type>::type;
   Cell<PlaneStoreLocal, TS> c;
   c.ps.pl = (float4*)smem;
   c.ps.lane = lane;
@@ -2875,12 +2884,22 @@ hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, i
   // the tet-major and site-major kernels start every pair from its tet's record
   if ((form == 0 || form == kFormTetCached || form == 1) && !a.tet_prep) return hipErrorInvalidValue;
   if (form == 0) {
-    const size_t lds = clip_plain_lds(a.pcap, a.tcap);
+    // With the vertices' distances kept beside the triangles the security test
+    // reads them instead of solving every vertex again for every bisector; where
+    // they cost a CU a resident wave, or do not fit, they are not kept (at the
+    // default caps 118 KB of LDS per wave instead of 94, one wave either way:
+    // 820k torus tets / 200,000 sites, whose re-clip ends in this launch, two
+    // iterations 34.9 -> 34.2 ms).
+    const size_t plain = clip_plain_lds(a.pcap, a.tcap), with_d2 = clip_plain_cached_lds(a.pcap, a.tcap);
+    constexpr size_t kLds = 160 * 1024;
+    const bool d2 = with_d2 <= kLds && kLds / with_d2 == kLds / plain;
+    const size_t lds = d2 ? with_d2 : plain;
     const dim3 grid(a.pair_list ? (unsigned)n_blocks : (unsigned)((a.n_pairs + 63) / 64)), block(64);
-    if (moments == 0 && acc_mode == 0) return launch_lds(k_clip_plain<0, 0, 0>, grid, block, lds, st, a);
-    if (moments == 0 && acc_mode == 1) return launch_lds(k_clip_plain<0, 1, 0>, grid, block, lds, st, a);
-    if (moments == 1 && acc_mode == 0) return launch_lds(k_clip_plain<1, 0, 0>, grid, block, lds, st, a);
-    return launch_lds(k_clip_plain<1, 1, 0>, grid, block, lds, st, a);
+    auto go = [&](auto kept, auto solved) { return launch_lds(d2 ? kept : solved, grid, block, lds, st, a); };
+    if (moments == 0 && acc_mode == 0) return go(k_clip_plain<0, 0, 2>, k_clip_plain<0, 0, 0>);
+    if (moments == 0 && acc_mode == 1) return go(k_clip_plain<0, 1, 2>, k_clip_plain<0, 1, 0>);
+    if (moments == 1 && acc_mode == 0) return go(k_clip_plain<1, 0, 2>, k_clip_plain<1, 0, 0>);
+    return go(k_clip_plain<1, 1, 2>, k_clip_plain<1, 1, 0>);
   }
   if (form == kFormTetCached) {
     if (a.tcap > 32) return hipErrorInvalidValue;
