@@ -1670,9 +1670,12 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
 // clipping.  A workgroup takes a site: one wavefront, or four on small problems
 // (a site has several hundred pairs, which one wave tests in a dozen trips).
 // It holds the site's first `depth` bisectors in LDS as planes n.x + w >= 0 on
-// the seed's side, each w raised by the test's margin: a tet whose four corners
-// all evaluate below zero lies beyond the bisector by more than the rounding
-// bound plus kCullMargin and its pair is empty.
+// the seed's side, each with a limit below zero: a tet whose four corners all
+// evaluate below it lies beyond the bisector by more than the rounding bound
+// plus kCullMargin and its pair is empty.  The limit of a bisector with an
+// infinite or NaN coefficient is -inf or NaN, and nothing is below that,
+// whatever such a plane evaluates to; a neighbour infinitely far by the FP32
+// distance ends the list, as every tet has a corner nearer than half of that.
 //
 // Which bisector empties a pair depends on where the tet lies: for each of the
 // 26 directions of a 3x3x3 neighbourhood the wave picks the two bisectors whose
@@ -1700,19 +1703,20 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ bool beyond(const float4& e, const P4 v[4]) {
+__device__ __forceinline__ bool beyond(const float4& e, float limit, const P4 v[4]) {
   float hi = -INFINITY;
 #pragma unroll
   for (int k = 0; k < 4; ++k) hi = fmaxf(hi, fmaf(e.z, v[k].z, fmaf(e.y, v[k].y, fmaf(e.x, v[k].x, e.w))));
-  return hi < 0.f;
+  return hi < limit;
 }
 
 template <int W>
 __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, const unsigned* pair_ids,
                                                       unsigned* out_ids, unsigned* pair_count) {
   extern __shared__ __align__(16) uint8_t smem[];
-  float4* eb = (float4*)smem;            // [depth] bisector (n, w + margin)
-  float* dd = (float*)(eb + depth);      // [depth] |z - s|^2
+  float4* eb = (float4*)smem;            // [depth] bisector (n, w)
+  float* lim = (float*)(eb + depth);     // [depth] limit of its test
+  float* dd = lim + depth;               // [depth] |z - s|^2
   uint32_t* first2 = (uint32_t*)(dd + depth);    // [27] the direction's two bisectors
   unsigned* survivors = (unsigned*)(first2 + 27);  // their number so far
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1751,24 +1755,27 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
     unsigned c0 = pb + 64 * wv;
     unsigned pair = pair_at(c0 + lane), pair1 = pair_at(c0 + 64 * W + lane);
     __syncthreads();  // the previous site's readers are done
-    int dv = depth;  // bisectors before the first invalid neighbour, which ends the clipping there
+    // bisectors before the first invalid neighbour, which ends the clipping
+    // there, or infinitely far one
+    int dv = depth;
     for (int v0 = 0; v0 < depth; v0 += 64) {
       const int v = v0 + lane;
       const int z = v < depth ? nbr[v] : 0;
       const bool bad = (unsigned)z >= (unsigned)a.n_sites;
-      const unsigned long long m = __ballot(bad);
+      const P4 zp = site_at(a, bad ? 0 : z);
+      const P4 d = sub3(zp, sp);
+      const float d2 = dot3(d, d);
+      const unsigned long long m = __ballot(v < depth && (bad || d2 == INFINITY));
       if (m && dv == depth) dv = v0 + __builtin_ctzll(m);
       if (v < depth && !bad && wv == 0) {
-        const P4 zp = site_at(a, z);
         const P4 eq = bisector(sp, zp);
-        const P4 d = sub3(zp, sp);
-        const float d2 = dot3(d, d);
         // the rounding of the evaluation (relative kCullRound of |n|_1 max|x| +
-        // |w|: one rounding of w and the margin, three of partial sums, all
-        // bounded by about that) plus kCullMargin in distance, times |n|
+        // |w|: three roundings of partial sums bounded by that) plus
+        // kCullMargin in distance, times |n|
         const float margin = fmaf(kCullRound, fmaf(fabsf(eq.x) + fabsf(eq.y) + fabsf(eq.z), a.max_coord, fabsf(eq.w)),
                                   kCullMargin * __builtin_amdgcn_sqrtf(d2));
-        eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w + margin);
+        eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w);
+        lim[v] = -margin;
         dd[v] = d2;
       }
     }
@@ -1827,9 +1834,10 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
       }
       bool open = live, culled = false;
       for (int q = 0; q < dv && __ballot(open) != 0; ++q) {
-        const bool cut = open && beyond(eb[q], t);
+        open = open && !(4.f * vmin2 <= dd[q]);
+        const bool cut = open && beyond(eb[q], lim[q], t);
         culled = culled || cut;
-        open = open && !cut && !(4.f * vmin2 <= dd[q]);
+        open = open && !cut;
       }
       record(pr, culled);
       const unsigned long long keep = __ballot(live && !culled);
@@ -1856,7 +1864,7 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
         const float t = 0.41421356f * fmaxf(fabsf(cx), fmaxf(fabsf(cy), fabsf(cz)));
         const int dir = 13 + (cx > t) - (cx < -t) + 3 * ((cy > t) - (cy < -t)) + 9 * ((cz > t) - (cz < -t));
         const uint32_t f = first2[dir];
-        const bool b0 = beyond(eb[f & 0xffffu], v), b1 = beyond(eb[f >> 16], v);
+        const bool b0 = beyond(eb[f & 0xffffu], lim[f & 0xffffu], v), b1 = beyond(eb[f >> 16], lim[f >> 16], v);
         culled = live && (b0 || b1);
       }
       pair = pair1;
@@ -2968,7 +2976,7 @@ hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* out_ids, 
 #endif
   const unsigned blocks =
       (unsigned)(kXcds * std::max(1, std::min((a.n_sites + kXcds - 1) / kXcds, VD_CULL_BLOCKS / kXcds)));
-  const size_t lds = 20 * (size_t)depth + 4 * (27 + 1);
+  const size_t lds = 24 * (size_t)depth + 4 * (27 + 1);
   if (out_ids != pair_ids)
     hipLaunchKernelGGL(k_cull_site<4>, dim3(blocks), dim3(256), lds + 4 * 4 * kCullQueue, st, a, depth, pair_ids,
                        out_ids, pair_count);
