@@ -1276,7 +1276,6 @@ __global__ __launch_bounds__(64) void k_clip_plain(ClipArgs a) {
 // others to finish).
 
 constexpr int kQueue = 128;           // ring of queued pair ids
-constexpr float kInvalidNbr = -1.f;   // table mark of an out-of-range neighbour id
 constexpr int kIdle = 0, kClipping = 1;  // lane states
 // Records of polytopes with more than kRecSplit vertices go to chunks of their
 // own, so that a wave of the volume pass (64 records of one chunk) runs over
