@@ -1669,12 +1669,14 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
 // clipping.  A workgroup takes a site: one wavefront, or four on small problems
 // (a site has several hundred pairs, which one wave tests in a dozen trips).
 // It holds the site's first `depth` bisectors in LDS as planes n.x + w >= 0 on
-// the seed's side, each with a limit below zero: a tet whose four corners all
-// evaluate below it lies beyond the bisector by more than the rounding bound
-// plus kCullMargin and its pair is empty.  The limit of a bisector with an
-// infinite or NaN coefficient is -inf or NaN, and nothing is below that,
-// whatever such a plane evaluates to; a neighbour infinitely far by the FP32
-// distance ends the list, as every tet has a corner nearer than half of that.
+// the seed's side: a tet whose four corners all evaluate below a limit, which
+// the tet's own largest coordinate gives, lies beyond the bisector by more than
+// the rounding bound plus kCullMargin and its pair is empty (a bound over the
+// mesh instead cost every tet as many bisectors as its farthest vertex, used or
+// not, asked for).  The limit of a bisector with an infinite or NaN coefficient
+// is -inf or NaN, and nothing is below that, whatever such a plane evaluates
+// to; a neighbour infinitely far by the FP32 distance ends the list, as every
+// tet has a corner nearer than half of that.
 //
 // Which bisector empties a pair depends on where the tet lies: for each of the
 // 26 directions of a 3x3x3 neighbourhood the wave picks the two bisectors whose
@@ -1702,11 +1704,21 @@ __device__ __forceinline__ void wave_fence() {
   __builtin_amdgcn_wave_barrier();
 }
 
-__device__ __forceinline__ bool beyond(const float4& e, float limit, const P4 v[4]) {
+__device__ __forceinline__ float coord_max(const P4 v[4]) {
+  float m = 0.f;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) m = fmaxf(m, fmaxf(fabsf(v[k].x), fmaxf(fabsf(v[k].y), fabsf(v[k].z))));
+  return m;
+}
+// m: |n|_1 and kCullMargin * |n| of bisector e; pmax: the corners' coord_max.
+// The limit is the rounding of the evaluation (relative kCullRound of |n|_1
+// max|x| + |w|: three roundings of partial sums bounded by that) plus
+// kCullMargin in distance, times |n|.
+__device__ __forceinline__ bool beyond(const float4& e, const float2& m, float pmax, const P4 v[4]) {
   float hi = -INFINITY;
 #pragma unroll
   for (int k = 0; k < 4; ++k) hi = fmaxf(hi, fmaf(e.z, v[k].z, fmaf(e.y, v[k].y, fmaf(e.x, v[k].x, e.w))));
-  return hi < limit;
+  return hi < -fmaf(kCullRound, fmaf(m.x, pmax, fabsf(e.w)), m.y);
 }
 
 template <int W>
@@ -1714,8 +1726,8 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
                                                       unsigned* out_ids, unsigned* pair_count) {
   extern __shared__ __align__(16) uint8_t smem[];
   float4* eb = (float4*)smem;            // [depth] bisector (n, w)
-  float* lim = (float*)(eb + depth);     // [depth] limit of its test
-  float* dd = lim + depth;               // [depth] |z - s|^2
+  float2* em = (float2*)(eb + depth);    // [depth] |n|_1, kCullMargin * |n|
+  float* dd = (float*)(em + depth);      // [depth] |z - s|^2
   uint32_t* first2 = (uint32_t*)(dd + depth);    // [27] the direction's two bisectors
   unsigned* survivors = (unsigned*)(first2 + 27);  // their number so far
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
@@ -1768,13 +1780,8 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
       if (m && dv == depth) dv = v0 + __builtin_ctzll(m);
       if (v < depth && !bad && wv == 0) {
         const P4 eq = bisector(sp, zp);
-        // the rounding of the evaluation (relative kCullRound of |n|_1 max|x| +
-        // |w|: three roundings of partial sums bounded by that) plus
-        // kCullMargin in distance, times |n|
-        const float margin = fmaf(kCullRound, fmaf(fabsf(eq.x) + fabsf(eq.y) + fabsf(eq.z), a.max_coord, fabsf(eq.w)),
-                                  kCullMargin * __builtin_amdgcn_sqrtf(d2));
         eb[v] = make_float4(eq.x, eq.y, eq.z, eq.w);
-        lim[v] = -margin;
+        em[v] = make_float2(fabsf(eq.x) + fabsf(eq.y) + fabsf(eq.z), kCullMargin * __builtin_amdgcn_sqrtf(d2));
         dd[v] = d2;
       }
     }
@@ -1831,10 +1838,11 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
         const P4 d = sub3(t[k], sp);
         vmin2 = fminf(vmin2, dot3(d, d));
       }
+      const float pmax = coord_max(t);
       bool open = live, culled = false;
       for (int q = 0; q < dv && __ballot(open) != 0; ++q) {
         open = open && !(4.f * vmin2 <= dd[q]);
-        const bool cut = open && beyond(eb[q], lim[q], t);
+        const bool cut = open && beyond(eb[q], em[q], pmax, t);
         culled = culled || cut;
         open = open && !cut;
       }
@@ -1862,8 +1870,9 @@ __global__ __launch_bounds__(64 * W) void k_cull_site(ClipArgs a, int depth, con
         const float cz = fmaf(-4.f, sp.z, (v[0].z + v[1].z) + (v[2].z + v[3].z));
         const float t = 0.41421356f * fmaxf(fabsf(cx), fmaxf(fabsf(cy), fabsf(cz)));
         const int dir = 13 + (cx > t) - (cx < -t) + 3 * ((cy > t) - (cy < -t)) + 9 * ((cz > t) - (cz < -t));
-        const uint32_t f = first2[dir];
-        const bool b0 = beyond(eb[f & 0xffffu], lim[f & 0xffffu], v), b1 = beyond(eb[f >> 16], lim[f >> 16], v);
+        const uint32_t f = first2[dir], f0 = f & 0xffffu, f1 = f >> 16;
+        const float pmax = coord_max(v);
+        const bool b0 = beyond(eb[f0], em[f0], pmax, v), b1 = beyond(eb[f1], em[f1], pmax, v);
         culled = live && (b0 || b1);
       }
       pair = pair1;
@@ -2975,7 +2984,7 @@ hipError_t cull_sites(const ClipArgs& a, unsigned* pair_ids, unsigned* out_ids, 
 #endif
   const unsigned blocks =
       (unsigned)(kXcds * std::max(1, std::min((a.n_sites + kXcds - 1) / kXcds, VD_CULL_BLOCKS / kXcds)));
-  const size_t lds = 24 * (size_t)depth + 4 * (27 + 1);
+  const size_t lds = 28 * (size_t)depth + 4 * (27 + 1);
   if (out_ids != pair_ids)
     hipLaunchKernelGGL(k_cull_site<4>, dim3(blocks), dim3(256), lds + 4 * 4 * kCullQueue, st, a, depth, pair_ids,
                        out_ids, pair_count);

@@ -25,7 +25,6 @@ struct ClipArgs {
   const unsigned* pair_ids;  // site-major form: n_pairs pair indices grouped by site
   const unsigned* pair_count;  // site-major and cell forms, optional: only the first pair_count[s]
                                // pairs of site s's range are clipped (cull_sites' survivors)
-  float max_coord;             // cull_sites: the mesh's largest |coordinate|
   const int* cell_status;      // cell form, optional: cull_sites keeps every pair of a site
                                // whose cell was not built (its pairs take the cell's status),
   const int* cell_nv;          // or whose cell's plane / triangle counts could overflow the

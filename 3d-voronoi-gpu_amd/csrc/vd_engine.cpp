@@ -824,8 +824,6 @@ int vd_clip_step(vd_ctx* ctx) {
   a.tet_prep = ctx->tet_prep.p;
   a.tet_knn = ctx->tet_knn.p;
   vd::set_tk(a, ctx->TK);
-  for (int x = 0; x < 3; ++x)
-    a.max_coord = std::max({a.max_coord, std::fabs(ctx->mesh_lo[x]), std::fabs(ctx->mesh_hi[x])});
   a.n_pairs = n_pairs;
   a.n_sites = n;
   a.pcap = c.pcap;
