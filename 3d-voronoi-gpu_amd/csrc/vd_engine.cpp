@@ -12,9 +12,9 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
-#include <climits>
 #include <cmath>
 #include <cstdarg>
+#include <cstdint>
 #include <cstdio>
 #include <cstring>
 #include <fstream>
@@ -47,6 +47,7 @@ struct DevBuf {
     p = nullptr;
     cap = 0;
   }
+  size_t bytes() const { return cap * sizeof(T); }
 };
 
 // Bisectors per site table of the site-major launch for K neighbours: by
@@ -216,7 +217,12 @@ struct vd_ctx {
   // site-major form: records of finished polytopes for the volume pass
   DevBuf<uint4> rec_meta;
   DevBuf<uint32_t> rec_tris;
-  long long more_records = LLONG_MAX;  // records beyond a tenth of the pairs, at most (vdi::limit_records)
+  // what units, p_ids2 and the records may take together (vdi::limit_scratch)
+  size_t scratch_limit = SIZE_MAX;
+  void release_records() {
+    rec_meta.release();
+    rec_tris.release();
+  }
   // pairs retried with deeper neighbour lists (srnr_k)
   DevBuf<unsigned> srnr_list;
   DevBuf<int> srnr_row_of, srnr_row_site;
@@ -898,10 +904,22 @@ int vd_clip_step(vd_ctx* ctx) {
     a.tcap_full = c.tcap;
     // (a depth at which every skipped pair is what the configured caps give)
     a.cull_depth = vd::exact_cull_depth(c.cull_depth, c.pcap, c.tcap);
+    // Pairs per work unit of the clipping: a wave serves two sites at a time, so
+    // units much below 64 pairs leave its lanes idle, and units that split most
+    // sites build their tables twice.  ms at 1M tets / 100,000 sites (10
+    // iterations), 820k torus tets (2), 48,000 tets / 2,000 sites (1): 32 pairs
+    // 93.9, 47.7, 1.12; 64 79.3, 44.9, 1.04; 128 75.3, 44.2, 1.06; 256 75.2,
+    // 44.5, 1.16; 1,024 75.3, 45.7, 1.24.
+    const int unit = n < kSplitSites ? 64 : 128;
+    const long long n_units = vd::max_site_units(n_pairs, n, unit);
+    // what is left for the survivors' list of the four-wave emptiness pass and
+    // the records, which results do not depend on
+    size_t left = ctx->scratch_limit;
+    left -= std::min(left, std::max((size_t)n_units * sizeof(uint4), ctx->units.bytes()));
     if (std::min(a.cull_depth, a.site_depth) > 0) {
       // the emptiness test as a pass of its own; the clipping takes the survivors
       unsigned* out = ctx->p_ids.p;
-      if (n <= kFourWaveSites) {
+      if (n <= kFourWaveSites && (size_t)n_pairs * sizeof(unsigned) <= left / 2) {
         VD_HIP(ctx->p_ids2.ensure(std::max(n_pairs, 1LL)), "alloc pairs");
         out = ctx->p_ids2.p;
       }
@@ -911,14 +929,8 @@ int vd_clip_step(vd_ctx* ctx) {
       a.pair_count = ctx->p_surv.p;
       a.cull_depth = 0;
     }
-    // Pairs per work unit of the clipping: a wave serves two sites at a time, so
-    // units much below 64 pairs leave its lanes idle, and units that split most
-    // sites build their tables twice.  ms at 1M tets / 100,000 sites (10
-    // iterations), 820k torus tets (2), 48,000 tets / 2,000 sites (1): 32 pairs
-    // 93.9, 47.7, 1.12; 64 79.3, 44.9, 1.04; 128 75.3, 44.2, 1.06; 256 75.2,
-    // 44.5, 1.16; 1,024 75.3, 45.7, 1.24.
-    const int unit = n < kSplitSites ? 64 : 128;
-    VD_HIP(ctx->units.ensure((size_t)vd::max_site_units(n_pairs, n, unit)), "alloc units");
+    left -= std::min(left, ctx->p_ids2.bytes());
+    VD_HIP(ctx->units.ensure((size_t)n_units), "alloc units");
     VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
     a.units = ctx->units.p;
     a.unit_count = ctx->counter(vd_ctx::kUnitCount);
@@ -929,9 +941,15 @@ int vd_clip_step(vd_ctx* ctx) {
       a.rec_chunk = n < kSplitSites ? 64 : 128;
       const long long more =
           (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
-      const long long ahead = 2LL * a.rec_chunk * std::min(kClipWaves, vd::max_site_units(n_pairs, n, unit));
-      const long long want = c.site_records > 0 ? std::min(c.site_records + 0LL, n_pairs)
-                                                : n_pairs / 10 + std::max(0LL, std::min(more, ctx->more_records)) + ahead;
+      const long long ahead = 2LL * a.rec_chunk * std::min(kClipWaves, n_units);
+      long long want = n_pairs / 10 + std::max(0LL, more) + ahead;
+      if (c.site_records > 0) {
+        want = std::min(c.site_records + 0LL, n_pairs);
+      } else {
+        const size_t rec_bytes = sizeof(uint4) + sizeof(uint32_t) * (size_t)vd::rec_stride(fast_tcap);
+        want = (long long)std::min((size_t)want, left / rec_bytes);
+        if (ctx->rec_meta.bytes() + ctx->rec_tris.bytes() > left) ctx->release_records();
+      }
       const unsigned cap = (unsigned)std::max(1LL, std::min(want, (long long)UINT32_MAX));
       VD_HIP(ctx->rec_meta.ensure(cap), "alloc records");
       VD_HIP(ctx->rec_tris.ensure((size_t)cap * vd::rec_stride(fast_tcap)), "alloc records");
@@ -1481,7 +1499,13 @@ namespace vdi {
 
 hipStream_t stream(vd_ctx* ctx) { return ctx->stream; }
 void set_error(vd_ctx* ctx, const char* msg) { ctx->err = msg; }
-void limit_records(vd_ctx* ctx, long long more) { ctx->more_records = more; }
+void limit_scratch(vd_ctx* ctx, size_t bytes) {
+  ctx->scratch_limit = bytes;
+  if (ctx->units.bytes() + ctx->p_ids2.bytes() + ctx->rec_meta.bytes() + ctx->rec_tris.bytes() <= bytes) return;
+  ctx->units.release();
+  ctx->p_ids2.release();
+  ctx->release_records();
+}
 
 int assemble(vd_ctx* ctx, const JobDev* jobs, int n) {
   if (!ctx || !jobs || n < 1) return VD_ERR_ARG;

@@ -53,8 +53,11 @@ double pieces_estimate(double n_tets, double n_sites);
 // re-clipped: 1.42 -> 1.10 ms and 2.0 -> 1.05 ms per clipping at 146,334 tets,
 // 16.8 -> 5.9 ms at 998,250).
 double records_per_tet(double n_tets, double n_sites, int TK);
-// At most `more` records beyond a tenth of the pairs in the automatic buffer.
-void limit_records(vd_ctx* ctx, long long more);
+// At most this many bytes for the site-major form's work units, the four-wave
+// emptiness pass's list and the automatic record buffer together.  The units
+// come first; the list and the records are cut to what is left, which changes
+// no result.  Gives back what an earlier batch left beyond the limit.
+void limit_scratch(vd_ctx* ctx, size_t bytes);
 // Vertex cap of the site-major launch under configuration c (its site_tcap,
 // or the automatic choice).
 int site_tcap_of(const vd_config& c);

@@ -152,6 +152,22 @@ struct vd_server {
     return code;
   }
 
+  size_t rec_bytes() const { return 16 + 4 * (size_t)vd::rec_stride(vdi::site_tcap_of(cfg)); }
+  // Bytes of the volume-pass records per tet that a job's footprint counts.
+  size_t rec_share() const {
+    return cfg.form == VD_FORM_SITE_MAJOR && cfg.site_records >= 0 ? rec_bytes() * (size_t)cfg.tet_k / 10 : 0;
+  }
+  // What the batch may take for records, work units and the emptiness pass's
+  // second list: the running jobs' shares, and what the budget has left or
+  // kFixedRecords records (25 MB at the automatic vertex cap, a fixed overhead
+  // outside the footprints) where that is more.
+  static constexpr size_t kFixedRecords = 262144;
+  size_t scratch(const Job* next = nullptr) {  // next: a job about to be admitted
+    size_t n = std::max(budget - used - (next ? next->bytes : 0), kFixedRecords * rec_bytes());
+    for (int id : running) n += rec_share() * (size_t)jobs[id].nt;
+    return n + (next ? rec_share() * (size_t)next->nt : 0);
+  }
+
   // Device bytes of a running job: its own buffers plus its share of the
   // batch's working memory (batch copies, the tets' start records, kNN
   // tables, grouped pairs, retry list, grid, the site-major form's
@@ -159,15 +175,11 @@ struct vd_server {
   size_t footprint(int nv, int nt, int ns) const {
     const size_t K = (size_t)cfg.site_k, TK = (size_t)cfg.tet_k;
     const size_t own = 16 * (size_t)nv + (16 + 48) * (size_t)nt + 16 * (size_t)ns + 4 * 256;
-    size_t rec = 0, cells = 0;
-    if (cfg.form == VD_FORM_SITE_MAJOR && cfg.site_records >= 0) {
-      const int ft = vdi::site_tcap_of(cfg);
-      rec = (16 + 4 * (size_t)vd::rec_stride(ft)) * TK / 10;
-    }
+    size_t cells = 0;
     // status, counts, radius, planes, triangles and the rebuild list per site
     if (cfg.form == VD_FORM_CELLS) cells = 20 + 16 * (size_t)cfg.pcap + 4 * (size_t)cfg.tcap;
     const size_t work =
-        16 * (size_t)nv + (16 + 48 + 16 * vd::kTetPrepWords + 12 * TK + rec + 8) * (size_t)nt +
+        16 * (size_t)nv + (16 + 48 + 16 * vd::kTetPrepWords + 12 * TK + rec_share() + 8) * (size_t)nt +
         (16 + 4 * K + 64 + cells) * (size_t)ns;
     return own + work;
   }
@@ -308,6 +320,7 @@ int vd_server_step(vd_server* s, int* n_running, int* n_pending) {
   while (!s->pending.empty()) {
     Job& j = s->jobs[s->pending.front()];
     if (s->used + j.bytes > s->budget) break;
+    vdi::limit_scratch(s->ctx, s->scratch(&j));  // (what it gives back, the job's buffers may need)
     const int rc = s->admit(j);
     if (rc != VD_OK) return rc;
     s->running.push_back(j.id);
@@ -326,12 +339,9 @@ int vd_server_step(vd_server* s, int* n_running, int* n_pending) {
         if (rc != VD_OK) return s->fail(rc, vd_ctx_error(s->ctx));
       }
       const std::vector<vdi::JobDev> cur = s->devs(s->running);
+      vdi::limit_scratch(s->ctx, s->scratch());
       int rc = vdi::assemble(s->ctx, cur.data(), (int)cur.size());
       if (rc != VD_OK) return s->fail(rc, vd_ctx_error(s->ctx));
-      // the jobs' footprints count one volume-pass record per ten pairs; more
-      // only from what the budget has left
-      vdi::limit_records(s->ctx, (long long)((s->budget - s->used) /
-                                             (16 + 4 * (size_t)vd::rec_stride(vdi::site_tcap_of(s->cfg)))));
       s->assembled = s->running;
       s->changed = false;
     }

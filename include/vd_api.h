@@ -298,6 +298,10 @@ int vd_kn_get_cell_counts(vd_kn* kn, int* out);
  * vd_server_step runs one Lloyd iteration over all running jobs as one batch
  * (vd_set_batch semantics, assembled on the device from the jobs' own
  * buffers).  A job's result is the one it gets alone with the same config.
+ * Working memory that results do not depend on (volume-pass records past one
+ * per ten pairs, work units, lists) is taken from what the budget has left, and
+ * given back as jobs are admitted; 262,144 records (25 MB at the automatic
+ * vertex cap) may be taken beyond the budget.
  * cfg->tet_k must be > 0 and every job needs more than site_k sites, so that
  * all jobs share K and TK.  No counterpart in the reference, which runs one
  * mesh per process (test_voronoi.cu:150-229). */
