@@ -125,12 +125,14 @@ __host__ __device__ inline int rec_stride(int tcap) { return (tcap + 3) & ~3; }
 
 // form: 0 tet-major, 1 site-major; moments: 0 reference, 1 robust;
 // acc_mode: 0 FP32 atomics, 1 FP64 pair sums + fixed-point site sums.
-// n_blocks: workgroups of the site-major form (0 = as many as stay resident),
-// and of the tet-major form when it runs over a.pair_list.  The site-major
+// n_blocks: workgroups of the site-major form (clip_site_blocks), and of the
+// tet-major form when it runs over a.pair_list.  The site-major
 // form with records (a.rec_meta) also launches their volume pass, unless
 // volume_pass is false (the caller then launches site_volume_pass).
 hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, int n_blocks, hipStream_t st,
                        bool volume_pass = true);
+// As many workgroups of the site-major launch with arguments a as stay resident.
+hipError_t clip_site_blocks(const ClipArgs& a, int moments, int acc_mode, int* n_blocks);
 // The volume pass over the records of a site-major launch with arguments a.
 hipError_t site_volume_pass(const ClipArgs& a, int moments, int acc_mode, hipStream_t st);
 

@@ -79,8 +79,6 @@ constexpr int kSplitSites = 8192;
 // iterations at 1,296 tets / 131 sites 3.05 ms against 3.16 with one, at 48,000
 // / 2,000 3.75 against 3.79 for six; at 82,944 / 8,294 7.24 against 7.12).
 constexpr int kFourWaveSites = 2048;
-// More waves than the GPU holds of the clipping kernel (9 per CU at most).
-constexpr long long kClipWaves = 2560;
 // kNN steps after the caller sets sites that do without the previous rows'
 // bounds (see vd_knn_step)
 constexpr int kHintAfter = 2;
@@ -934,6 +932,9 @@ int vd_clip_step(vd_ctx* ctx) {
     VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
     a.units = ctx->units.p;
     a.unit_count = ctx->counter(vd_ctx::kUnitCount);
+    int resident = 0;  // (a launch of more workgroups has no units left for the others)
+    VD_HIP(vd::clip_site_blocks(a, c.moments, c.accum, &resident), "clip");
+    if (blocks <= 0) blocks = resident;
     if (c.site_records >= 0) {
       // automatic: the estimate, plus the slots that the waves reserve ahead (a
       // chunk of each size class per wave; smaller chunks where every wave has
@@ -941,7 +942,7 @@ int vd_clip_step(vd_ctx* ctx) {
       a.rec_chunk = n < kSplitSites ? 64 : 128;
       const long long more =
           (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
-      const long long ahead = 2LL * a.rec_chunk * std::min(kClipWaves, n_units);
+      const long long ahead = 2LL * a.rec_chunk * std::min<long long>(std::min(blocks, resident), n_units);
       long long want = n_pairs / 10 + std::max(0LL, more) + ahead;
       if (c.site_records > 0) {
         want = std::min(c.site_records + 0LL, n_pairs);
