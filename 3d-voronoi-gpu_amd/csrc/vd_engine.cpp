@@ -72,9 +72,14 @@ constexpr int kFreshSiteDepth = 64;
 // 48,000 0.60 / 0.69, 82,944 (386k pieces) 0.80 / 0.77, 146,334 1.25 / 1.14.
 constexpr double kWidePieces = 256e3;
 constexpr int kWideDepth = 96, kWideTcap = 32;
-// Below this many sites the clipping's work units and the records that a wave
-// reserves at a time are smaller.
-constexpr int kSplitSites = 8192;
+// Below this many sites the clipping's work units are of 64 pairs, so that there
+// are several for every wave, and from it on of 128.  Clipping us of four
+// iterations, 64 against 128: 600 sites (6,000 tets) 985 / 1,063, 1,500 (82,944)
+// 1,566 / 1,617, 2,000 (48,000) 1,511 / 1,573, 2,000 (511,104) 3,455 / 3,374;
+// 3,001 (29,478) 1,590 / 1,568, 3,500 (48,000) 1,869 / 1,805, 4,000 (82,944)
+// 2,347 / 2,392, 4,000 (511,104) 4,080 / 4,000, 4,800 (48,000) 2,129 / 2,043,
+// 8,294 (82,944) 2,870 / 2,816.
+constexpr int kSplitSites = 2500;
 // Up to this many sites the emptiness pass takes each with four waves (ten
 // iterations at 1,296 tets / 131 sites 3.05 ms against 3.16 with one, at 48,000
 // / 2,000 3.75 against 3.79 for six; at 82,944 / 8,294 7.24 against 7.12).
@@ -880,7 +885,8 @@ int vd_clip_step(vd_ctx* ctx) {
     a.site_counter = ctx->counter(vd_ctx::kUnitCounter);
     int fast_tcap = vdi::site_tcap_of(c);
     a.site_depth = site_depth_of(c, ctx->K);
-    wide = c.site_tcap == 0 && c.site_depth == 0 && vdi::pieces_estimate(ctx->n_tets, n) <= kWidePieces;
+    const double pieces = vdi::pieces_estimate(ctx->n_tets, n);
+    wide = c.site_tcap == 0 && c.site_depth == 0 && pieces <= kWidePieces;
     if (wide) {
       fast_tcap = std::min(c.tcap, kWideTcap);
       a.site_depth = std::min(kWideDepth, ctx->K);
@@ -936,10 +942,13 @@ int vd_clip_step(vd_ctx* ctx) {
     VD_HIP(vd::clip_site_blocks(a, c.moments, c.accum, &resident), "clip");
     if (blocks <= 0) blocks = resident;
     if (c.site_records >= 0) {
-      // automatic: the estimate, plus the slots that the waves reserve ahead (a
-      // chunk of each size class per wave; smaller chunks where every wave has
-      // few pairs)
-      a.rec_chunk = n < kSplitSites ? 64 : 128;
+      // automatic: the estimate, plus the slots that the waves reserve ahead, a
+      // chunk of each size class per wave.  The volume pass reads the unused
+      // ones too, so the chunks are smaller where every wave has few pieces: us
+      // of four iterations, 64 against 128, 138k pieces 1,568 / 1,647, 169k
+      // 2,135 / 2,224, 223k 2,043 / 2,094; 294k 2,392 / 2,376, 386k 2,816 /
+      // 2,799, 2.4M 9,270 / 9,220.
+      a.rec_chunk = pieces <= kWidePieces ? 64 : 128;
       const long long more =
           (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
       const long long ahead = 2LL * a.rec_chunk * std::min<long long>(std::min(blocks, resident), n_units);
