@@ -938,9 +938,16 @@ int vd_clip_step(vd_ctx* ctx) {
     VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
     a.units = ctx->units.p;
     a.unit_count = ctx->counter(vd_ctx::kUnitCount);
-    int resident = 0;  // (a launch of more workgroups has no units left for the others)
-    VD_HIP(vd::clip_site_blocks(a, c.moments, c.accum, &resident), "clip");
-    if (blocks <= 0) blocks = resident;
+    // the workgroups that stay resident (of more, the others find no unit left),
+    // for the records at the depth of moved sites, so that the second iteration
+    // needs no larger buffer than the first
+    vd::ClipArgs moved = a;
+    if (!wide) moved.site_depth = site_depth_of(c, ctx->K);
+    int resident = 0;
+    VD_HIP(vd::clip_site_blocks(moved, c.moments, c.accum, &resident), "clip");
+    const long long waves = std::min<long long>(blocks > 0 ? blocks : resident, resident);
+    if (blocks <= 0 && moved.site_depth == a.site_depth) blocks = resident;
+    if (blocks <= 0) VD_HIP(vd::clip_site_blocks(a, c.moments, c.accum, &blocks), "clip");
     if (c.site_records >= 0) {
       // automatic: the estimate, plus the slots that the waves reserve ahead, a
       // chunk of each size class per wave.  The volume pass reads the unused
@@ -951,7 +958,7 @@ int vd_clip_step(vd_ctx* ctx) {
       a.rec_chunk = pieces <= kWidePieces ? 64 : 128;
       const long long more =
           (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
-      const long long ahead = 2LL * a.rec_chunk * std::min<long long>(std::min(blocks, resident), n_units);
+      const long long ahead = 2LL * a.rec_chunk * std::min(waves, n_units);
       long long want = n_pairs / 10 + std::max(0LL, more) + ahead;
       if (c.site_records > 0) {
         want = std::min(c.site_records + 0LL, n_pairs);

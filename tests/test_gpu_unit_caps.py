@@ -1,9 +1,12 @@
 """The site-major clipping's work units at vertex caps and table depths that
 leave pairs to the re-clip (the automatic ones of large problems, and smaller
 ones, with more resident waves), every pair against the oracle bit for bit."""
+import ctypes
+
 import numpy as np
 import pytest
 from conftest import oracle_knn, problem
+from test_gpu_knn import _Hip
 
 pytestmark = pytest.mark.gpu
 
@@ -35,3 +38,25 @@ def test_units_at_small_caps(vdn, O, n, ns, tk, cfg):
             np.testing.assert_array_equal(e.moments(), r["site_vals"])
             hist = e.status_hist()
             assert [hist[k] for k in vdn.STATUS_NAMES] == np.bincount(r["pair_status"], minlength=7).tolist()
+
+
+@pytest.mark.parametrize("n,ns", [(10, 600), (24, 8294)])
+def test_second_iteration_allocates_nothing(vdn, n, ns):
+    """(An iteration that allocated could not be captured in a graph.)"""
+    hip = _Hip()
+
+    def free():
+        a, b = ctypes.c_size_t(), ctypes.c_size_t()
+        assert hip.L.hipDeviceSynchronize() == 0
+        assert hip.L.hipMemGetInfo(ctypes.byref(a), ctypes.byref(b)) == 0
+        return a.value
+
+    verts, tets, sites = problem("cube", n, ns)
+    for moments in ("reference", "robust"):
+        with vdn.Engine(tet_k=20, accum="f64", moments=moments) as e:
+            e.set_mesh(verts, tets)
+            e.set_sites(sites)
+            e.lloyd(1)
+            before = free()
+            e.lloyd(2)
+            assert free() == before
