@@ -84,6 +84,9 @@ constexpr int kSplitSites = 2500;
 // iterations at 1,296 tets / 131 sites 3.05 ms against 3.16 with one, at 48,000
 // / 2,000 3.75 against 3.79 for six; at 82,944 / 8,294 7.24 against 7.12).
 constexpr int kFourWaveSites = 2048;
+// New record and list buffers of up to this size are made without a look at the
+// device's free memory (which takes some 50 us of host time).
+constexpr size_t kCheckedGrowth = (size_t)256 << 20;
 // kNN steps after the caller sets sites that do without the previous rows'
 // bounds (see vd_knn_step)
 constexpr int kHintAfter = 2;
@@ -222,6 +225,10 @@ struct vd_ctx {
   DevBuf<uint32_t> rec_tris;
   // what units, p_ids2 and the records may take together (vdi::limit_scratch)
   size_t scratch_limit = SIZE_MAX;
+  // the present meshes leave the device no room for the records of all estimated
+  // pieces and the emptiness pass's second list
+  bool tight = false;
+  size_t record_bytes() const { return rec_meta.bytes() + rec_tris.bytes(); }
   void release_records() {
     rec_meta.release();
     rec_tris.release();
@@ -298,6 +305,35 @@ hipError_t record_phase(vd_ctx* ctx, int phase, hipStream_t st = nullptr) {
   return ctx->record(phase, st ? st : ctx->stream);
 }
 
+
+// Fits the emptiness pass's second list (two_lists, of `list` bytes) and the
+// records (of rec_bytes each) to what there is room for; results depend on
+// neither.  Under vdi::limit_scratch: the units come first, then the list where
+// it takes at most half of the rest, then the records.  On the device: more than
+// kCheckedGrowth of new buffers only where that leaves the step's later lists
+// room; else no list and at most `fewer` records (the pieces past them are
+// integrated in place or re-clipped).
+int fit_scratch(vd_ctx* ctx, size_t units, size_t list, size_t rec_bytes, long long fewer, bool* two_lists,
+                long long* records) {
+  size_t left = ctx->scratch_limit;
+  left -= std::min(left, std::max(units, ctx->units.bytes()));
+  *two_lists = *two_lists && list <= left / 2;
+  left -= std::min(left, std::max(*two_lists ? list : 0, ctx->p_ids2.bytes()));
+  if (ctx->cfg.site_records == 0) *records = (long long)std::min((size_t)*records, left / rec_bytes);
+  if (ctx->record_bytes() > left) ctx->release_records();
+  const size_t held = ctx->record_bytes(), rec = (size_t)*records * rec_bytes;
+  const size_t grow = (rec > held ? rec : 0) + (*two_lists && ctx->p_ids2.bytes() < list ? list : 0);
+  if (!ctx->tight && grow > kCheckedGrowth) {
+    size_t free = 0, total = 0;
+    VD_HIP(hipMemGetInfo(&free, &total), "device memory");
+    ctx->tight = grow + 3 * list > free + held + ctx->p_ids2.bytes();
+  }
+  if (ctx->tight) {
+    *records = std::min(*records, fewer);
+    *two_lists = false;
+  }
+  return VD_OK;
+}
 
 int check_config(vd_ctx* ctx, const vd_config& c) {
   if (c.site_k < 1 || c.site_k > 256) return ctx->fail(VD_ERR_ARG, "site_k must be in [1,256], got %d", c.site_k);
@@ -544,6 +580,7 @@ namespace {
 // Uploads vertices, tets (global vertex ids, validated by the caller) and the
 // per-tet corner records; sets the mesh bounding box.
 int load_mesh(vd_ctx* ctx, const float* verts_xyz, int n_verts, const int32_t* tets, int n_tets) {
+  ctx->tight = false;
   for (int a = 0; a < 3; ++a) {
     ctx->mesh_lo[a] = n_verts ? verts_xyz[a] : 0.f;
     ctx->mesh_hi[a] = n_verts ? verts_xyz[a] : 0.f;
@@ -916,28 +953,9 @@ int vd_clip_step(vd_ctx* ctx) {
     // 44.5, 1.16; 1,024 75.3, 45.7, 1.24.
     const int unit = n < kSplitSites ? 64 : 128;
     const long long n_units = vd::max_site_units(n_pairs, n, unit);
-    // what is left for the survivors' list of the four-wave emptiness pass and
-    // the records, which results do not depend on
-    size_t left = ctx->scratch_limit;
-    left -= std::min(left, std::max((size_t)n_units * sizeof(uint4), ctx->units.bytes()));
-    if (std::min(a.cull_depth, a.site_depth) > 0) {
-      // the emptiness test as a pass of its own; the clipping takes the survivors
-      unsigned* out = ctx->p_ids.p;
-      if (n <= kFourWaveSites && (size_t)n_pairs * sizeof(unsigned) <= left / 2) {
-        VD_HIP(ctx->p_ids2.ensure(std::max(n_pairs, 1LL)), "alloc pairs");
-        out = ctx->p_ids2.p;
-      }
-      VD_HIP(ctx->p_surv.ensure(n), "alloc pairs");
-      VD_HIP(vd::cull_sites(a, ctx->p_ids.p, out, ctx->p_surv.p, ctx->stream), "cull");
-      a.pair_ids = out;
-      a.pair_count = ctx->p_surv.p;
-      a.cull_depth = 0;
-    }
-    left -= std::min(left, ctx->p_ids2.bytes());
-    VD_HIP(ctx->units.ensure((size_t)n_units), "alloc units");
-    VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
-    a.units = ctx->units.p;
-    a.unit_count = ctx->counter(vd_ctx::kUnitCount);
+    const size_t list = (size_t)std::max(n_pairs, 1LL) * sizeof(unsigned);
+    const bool cull = std::min(a.cull_depth, a.site_depth) > 0;
+    bool two_lists = cull && n <= kFourWaveSites;
     // the workgroups that stay resident (of more, the others find no unit left),
     // for the records at the depth of moved sites, so that the second iteration
     // needs no larger buffer than the first
@@ -948,32 +966,45 @@ int vd_clip_step(vd_ctx* ctx) {
     const long long waves = std::min<long long>(blocks > 0 ? blocks : resident, resident);
     if (blocks <= 0 && moved.site_depth == a.site_depth) blocks = resident;
     if (blocks <= 0) VD_HIP(vd::clip_site_blocks(a, c.moments, c.accum, &blocks), "clip");
+    // records: the estimate, plus the slots that the waves reserve ahead, a chunk
+    // of each size class per wave.  The volume pass reads the unused ones too, so
+    // the chunks are smaller where every wave has few pieces: us of four
+    // iterations, 64 against 128, 138k pieces 1,568 / 1,647, 169k 2,135 / 2,224,
+    // 223k 2,043 / 2,094; 294k 2,392 / 2,376, 386k 2,816 / 2,799, 2.4M 9,270 /
+    // 9,220.
+    a.rec_chunk = pieces <= kWidePieces ? 64 : 128;
+    const int stride = vd::rec_stride(fast_tcap);
+    const long long ahead = 2LL * a.rec_chunk * std::min(waves, n_units);
+    const long long tenth = n_pairs / 10;
+    long long records = 0;
+    if (c.site_records > 0) records = std::min(c.site_records + 0LL, n_pairs);
+    if (c.site_records == 0)
+      records = std::max(tenth, (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets)) + ahead;
+    const int rc = fit_scratch(ctx, (size_t)n_units * sizeof(uint4), list, sizeof(uint4) + sizeof(uint32_t) * stride,
+                               c.site_records == 0 ? tenth + ahead : records, &two_lists, &records);
+    if (rc != VD_OK) return rc;
+    if (cull) {
+      // the emptiness test as a pass of its own; the clipping takes the survivors
+      if (two_lists) VD_HIP(ctx->p_ids2.ensure(list / sizeof(unsigned)), "alloc pairs");
+      unsigned* out = two_lists ? ctx->p_ids2.p : ctx->p_ids.p;
+      VD_HIP(ctx->p_surv.ensure(n), "alloc pairs");
+      VD_HIP(vd::cull_sites(a, ctx->p_ids.p, out, ctx->p_surv.p, ctx->stream), "cull");
+      a.pair_ids = out;
+      a.pair_count = ctx->p_surv.p;
+      a.cull_depth = 0;
+    }
+    VD_HIP(ctx->units.ensure((size_t)n_units), "alloc units");
+    VD_HIP(vd::site_units(a, unit, ctx->units.p, ctx->counter(vd_ctx::kUnitCount), ctx->stream), "units");
+    a.units = ctx->units.p;
+    a.unit_count = ctx->counter(vd_ctx::kUnitCount);
     if (c.site_records >= 0) {
-      // automatic: the estimate, plus the slots that the waves reserve ahead, a
-      // chunk of each size class per wave.  The volume pass reads the unused
-      // ones too, so the chunks are smaller where every wave has few pieces: us
-      // of four iterations, 64 against 128, 138k pieces 1,568 / 1,647, 169k
-      // 2,135 / 2,224, 223k 2,043 / 2,094; 294k 2,392 / 2,376, 386k 2,816 /
-      // 2,799, 2.4M 9,270 / 9,220.
-      a.rec_chunk = pieces <= kWidePieces ? 64 : 128;
-      const long long more =
-          (long long)(vdi::records_per_tet(ctx->n_tets, n, ctx->TK) * ctx->n_tets) - n_pairs / 10;
-      const long long ahead = 2LL * a.rec_chunk * std::min(waves, n_units);
-      long long want = n_pairs / 10 + std::max(0LL, more) + ahead;
-      if (c.site_records > 0) {
-        want = std::min(c.site_records + 0LL, n_pairs);
-      } else {
-        const size_t rec_bytes = sizeof(uint4) + sizeof(uint32_t) * (size_t)vd::rec_stride(fast_tcap);
-        want = (long long)std::min((size_t)want, left / rec_bytes);
-        if (ctx->rec_meta.bytes() + ctx->rec_tris.bytes() > left) ctx->release_records();
-      }
-      const unsigned cap = (unsigned)std::max(1LL, std::min(want, (long long)UINT32_MAX));
-      VD_HIP(ctx->rec_meta.ensure(cap), "alloc records");
-      VD_HIP(ctx->rec_tris.ensure((size_t)cap * vd::rec_stride(fast_tcap)), "alloc records");
+      const long long cap = std::max(1LL, std::min(records, (long long)UINT32_MAX));
+      VD_HIP(ctx->rec_meta.ensure((size_t)cap), "alloc records");
+      VD_HIP(ctx->rec_tris.ensure((size_t)cap * stride), "alloc records");
       a.rec_meta = ctx->rec_meta.p;
       a.rec_tris = ctx->rec_tris.p;
       a.rec_count = ctx->counter(vd_ctx::kRecCount);
-      a.rec_cap = cap;
+      a.rec_cap = (unsigned)cap;
     }
   } else {
     VD_HIP(record_phase(ctx, (2)), "event");
@@ -1518,7 +1549,7 @@ hipStream_t stream(vd_ctx* ctx) { return ctx->stream; }
 void set_error(vd_ctx* ctx, const char* msg) { ctx->err = msg; }
 void limit_scratch(vd_ctx* ctx, size_t bytes) {
   ctx->scratch_limit = bytes;
-  if (ctx->units.bytes() + ctx->p_ids2.bytes() + ctx->rec_meta.bytes() + ctx->rec_tris.bytes() <= bytes) return;
+  if (ctx->units.bytes() + ctx->p_ids2.bytes() + ctx->record_bytes() <= bytes) return;
   ctx->units.release();
   ctx->p_ids2.release();
   ctx->release_records();
@@ -1528,6 +1559,7 @@ int assemble(vd_ctx* ctx, const JobDev* jobs, int n) {
   if (!ctx || !jobs || n < 1) return VD_ERR_ARG;
   VD_HIP(hipSetDevice(ctx->device), "set device");
   ctx->drop_graph();
+  ctx->tight = false;
   std::vector<vd_ctx::Inst> in((size_t)n);
   long long V = 0, T = 0, S = 0;
   for (int i = 0; i < n; ++i) {

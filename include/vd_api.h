@@ -98,7 +98,8 @@ typedef struct vd_config {
                          per vertex of the launch cap, rounded up to 4 vertices); past it a
                          lane computes its volume in place, so results do not depend on it;
                          0 = automatic (the larger of a tenth of the pairs and 1.3 times the
-                         estimated pieces, plus what the waves reserve ahead), -1 = every volume in place */
+                         estimated pieces, plus what the waves reserve ahead; a tenth where
+                         the device has no room for more), -1 = every volume in place */
   int site_depth;     /* site-major form: bisectors per site table of the launch; a pair that
                          needs more is recomputed from scratch at site_k by the retry pass,
                          so results do not depend on it; 0 = automatic (40, and 64 for the
