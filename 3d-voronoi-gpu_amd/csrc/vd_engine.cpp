@@ -319,8 +319,10 @@ int fit_scratch(vd_ctx* ctx, size_t units, size_t list, size_t rec_bytes, long l
   left -= std::min(left, std::max(units, ctx->units.bytes()));
   *two_lists = *two_lists && list <= left / 2;
   left -= std::min(left, std::max(*two_lists ? list : 0, ctx->p_ids2.bytes()));
-  if (ctx->cfg.site_records == 0) *records = (long long)std::min((size_t)*records, left / rec_bytes);
-  if (ctx->record_bytes() > left) ctx->release_records();
+  if (ctx->cfg.site_records == 0) {  // (a given number is taken as it is)
+    *records = (long long)std::min((size_t)*records, left / rec_bytes);
+    if (ctx->record_bytes() > left) ctx->release_records();
+  }
   const size_t held = ctx->record_bytes(), rec = (size_t)*records * rec_bytes;
   const size_t grow = (rec > held ? rec : 0) + (*two_lists && ctx->p_ids2.bytes() < list ? list : 0);
   if (!ctx->tight && grow > kCheckedGrowth) {

@@ -76,3 +76,19 @@ def test_records_within_the_jobs_shares(vdn, n, ns):
     used, _ = _used(vdn, hip, budget, [jobs])
     share = sum(len(p[1]) for p in jobs) * CFG["tet_k"] // 10 * REC
     assert used - without <= share + 262144 * REC + 8 * MB
+
+
+def test_given_records_are_kept(vdn):
+    """A given number of records above the limit: taken as it is, with the same
+    memory at each step."""
+    hip = _Hip()
+    p = problem("cube", 20, 2000)
+    with vdn.Server(budget_bytes=_job_bytes(vdn, p) + MB, **{**CFG, "site_records": 900000}) as s:
+        j = s.submit(*p, 8)
+        s.step()
+        held = _free(hip)
+        for _ in range(6):
+            s.step()
+            assert _free(hip) == held
+        assert s.step() == (0, 0)
+        np.testing.assert_array_equal(s.result(j), _alone(vdn, p, 8))
