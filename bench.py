@@ -406,8 +406,9 @@ def main():
         sets = chain_sites(native, verts, tets, sites, min(CHAIN, args.steps), **FAST)
         flops, base = count_flops(verts, tets, sets)
         # the three launches of the clipping (emptiness pass, clipping, volume
-        # pass) on the engine's stream: the clip phase minus the exposed part
-        # of the overflow re-clip beside the volume pass
+        # pass): the clip phase minus what of the overflow re-clip is left when
+        # the volume pass ends; the re-clip runs beside the volume pass, so the
+        # time contains what it takes from it
         kern_ms = [tl[j]["clip_ms"] - tl[j]["overflow_ms"] for j in range(len(tl))]
         f_timed = [flops[j % CHAIN] for j in range(len(tl))]
         achieved = sum(f_timed) / (sum(kern_ms) / 1e3) / 1e12

@@ -121,9 +121,11 @@ typedef struct vd_timing {
   float clip_ms;   /* clipping + per-site accumulation */
   float update_ms; /* Lloyd update */
   float total_ms;  /* whole iteration */
-  float overflow_ms; /* part of clip_ms: re-clipping of the pairs that overflowed the
-                        site-major launch's vertex cap, at the configured caps, and of the
-                        pairs retried with srnr_k neighbours */
+  float overflow_ms; /* part of clip_ms after the clipping and its volume pass have ended:
+                        what is left then of the re-clip of the pairs that overflowed the
+                        site-major launch's vertex cap (which runs beside the volume pass and
+                        is not counted while it does), and the pairs retried with srnr_k
+                        neighbours */
 } vd_timing;
 
 typedef struct vd_ctx vd_ctx;
