@@ -2877,29 +2877,21 @@ static hipError_t launch_lds(Kern k, dim3 grid, dim3 block, size_t lds, hipStrea
   return hipGetLastError();
 }
 
-// The site-major kernel is persistent (waves take work units from a counter): by
-// default one workgroup per slot the device can keep resident (clip_site_blocks).
-static auto site_kernel(int moments, int acc_mode) -> void (*)(ClipArgs) {
-  if (moments == 0) return acc_mode == 0 ? k_clip_site<0, 0> : k_clip_site<0, 1>;
-  return acc_mode == 0 ? k_clip_site<1, 0> : k_clip_site<1, 1>;
-}
-
-static size_t site_lds(const ClipArgs& a) {
-  return clip_site_lds(a.site_depth > 0 ? std::min(a.site_depth, a.K) : a.K, a.tcap);
-}
-
-hipError_t clip_site_blocks(const ClipArgs& a, int moments, int acc_mode, int* n_blocks) {
-  const size_t lds = site_lds(a);
-  auto k = site_kernel(moments, acc_mode);
-  int per_cu = 0, dev = 0, cus = 0;
-  hipError_t e;
-  if ((e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds)) != hipSuccess)
-    return e;
-  if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds)) != hipSuccess) return e;
-  if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
-  if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
-  *n_blocks = std::max(1, per_cu * cus);
-  return hipSuccess;
+// The site-major kernel is persistent (waves take sites from a counter): by
+// default one workgroup per slot the device can keep resident.
+template <class Kern>
+static hipError_t launch_site(Kern k, int n_blocks, size_t lds, hipStream_t st, const ClipArgs& a) {
+  hipError_t e = hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+  if (e != hipSuccess) return e;
+  if (n_blocks <= 0) {
+    int per_cu = 0, dev = 0, cus = 0;
+    if ((e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k, 64, lds)) != hipSuccess) return e;
+    if ((e = hipGetDevice(&dev)) != hipSuccess) return e;
+    if ((e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev)) != hipSuccess) return e;
+    n_blocks = std::max(1, per_cu * cus);
+  }
+  hipLaunchKernelGGL(k, dim3((unsigned)n_blocks), dim3(64), lds, st, a);
+  return hipGetLastError();
 }
 
 hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, int n_blocks, hipStream_t st,
@@ -2941,9 +2933,16 @@ hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, i
   // polytopes it cannot hand to the volume pass go to the retry list
   if (moments == 1 && (!a.retry_list || !a.retry_count)) return hipErrorInvalidValue;
   if (a.site_depth > 0 && a.site_depth < a.K && (!a.retry_list || !a.retry_count)) return hipErrorInvalidValue;
-  if (n_blocks < 1) return hipErrorInvalidValue;
-  const hipError_t e =
-      launch_lds(site_kernel(moments, acc_mode), dim3((unsigned)n_blocks), dim3(64), site_lds(a), st, a);
+  const size_t lds = clip_site_lds(a.site_depth > 0 ? std::min(a.site_depth, a.K) : a.K, a.tcap);
+  hipError_t e;
+  if (moments == 0 && acc_mode == 0)
+    e = launch_site(k_clip_site<0, 0>, n_blocks, lds, st, a);
+  else if (moments == 0 && acc_mode == 1)
+    e = launch_site(k_clip_site<0, 1>, n_blocks, lds, st, a);
+  else if (moments == 1 && acc_mode == 0)
+    e = launch_site(k_clip_site<1, 0>, n_blocks, lds, st, a);
+  else
+    e = launch_site(k_clip_site<1, 1>, n_blocks, lds, st, a);
   if (e != hipSuccess || !volume_pass) return e;
   return site_volume_pass(a, moments, acc_mode, st);
 }

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
+
 namespace vd {
 
 struct ClipArgs {
@@ -120,19 +122,22 @@ hipError_t cells_launch(const ClipArgs& a, const CellStore& cs, int moments, int
                         int fast_tcap = 0);
 // LDS of the site-major kernel with `depth` bisectors per site table.
 size_t clip_site_lds(int depth, int tcap);
+// Waves of it that a CU holds at most: by LDS (allocated 512 bytes at a time), and
+// 16 by the registers (109 to 116 VGPRs).
+inline int clip_site_waves_per_cu(int depth, int tcap) {
+  return (int)std::min<size_t>(16, 160 * 1024 / ((clip_site_lds(depth, tcap) + 511) & ~(size_t)511));
+}
 // Triangle words per record of the site-major form's volume pass.
 __host__ __device__ inline int rec_stride(int tcap) { return (tcap + 3) & ~3; }
 
 // form: 0 tet-major, 1 site-major; moments: 0 reference, 1 robust;
 // acc_mode: 0 FP32 atomics, 1 FP64 pair sums + fixed-point site sums.
-// n_blocks: workgroups of the site-major form (clip_site_blocks), and of the
-// tet-major form when it runs over a.pair_list.  The site-major
+// n_blocks: workgroups of the site-major form (0 = as many as stay resident),
+// and of the tet-major form when it runs over a.pair_list.  The site-major
 // form with records (a.rec_meta) also launches their volume pass, unless
 // volume_pass is false (the caller then launches site_volume_pass).
 hipError_t clip_launch(const ClipArgs& a, int form, int moments, int acc_mode, int n_blocks, hipStream_t st,
                        bool volume_pass = true);
-// As many workgroups of the site-major launch with arguments a as stay resident.
-hipError_t clip_site_blocks(const ClipArgs& a, int moments, int acc_mode, int* n_blocks);
 // The volume pass over the records of a site-major launch with arguments a.
 hipError_t site_volume_pass(const ClipArgs& a, int moments, int acc_mode, hipStream_t st);
 

@@ -72,14 +72,15 @@ constexpr int kFreshSiteDepth = 64;
 // 48,000 0.60 / 0.69, 82,944 (386k pieces) 0.80 / 0.77, 146,334 1.25 / 1.14.
 constexpr double kWidePieces = 256e3;
 constexpr int kWideDepth = 96, kWideTcap = 32;
-// Below this many sites the clipping's work units are of 64 pairs, so that there
-// are several for every wave, and from it on of 128.  Clipping us of four
-// iterations, 64 against 128: 600 sites (6,000 tets) 985 / 1,063, 1,500 (82,944)
-// 1,566 / 1,617, 2,000 (48,000) 1,511 / 1,573, 2,000 (511,104) 3,455 / 3,374;
-// 3,001 (29,478) 1,590 / 1,568, 3,500 (48,000) 1,869 / 1,805, 4,000 (82,944)
-// 2,347 / 2,392, 4,000 (511,104) 4,080 / 4,000, 4,800 (48,000) 2,129 / 2,043,
-// 8,294 (82,944) 2,870 / 2,816.
-constexpr int kSplitSites = 2500;
+// From this many sites on the clipping's work units are of 128 pairs, below it of
+// 64, which give every wave several.  Clipping us of four iterations, 64 against
+// 128: 8,294 sites (82,944 tets) 2,870 / 2,816, 13,171 (131,712) 3,660 / 3,530,
+// 16,000 (511,104) 6,340 / 6,010, 42,592 (511,104) 10,430 / 9,230; 600 sites (6,000)
+// 985 / 1,063, 1,500 (82,944) 1,566 / 1,617, 2,000 (48,000) 1,511 / 1,573.  Between
+// 2,500 and the line it is the survivors per site that decide, some 70 to 100 for
+// 128 (4,800 sites, 48,000 tets, 2,129 / 2,043: 64 leaves a small second unit), 150
+// for 64 (4,000, 82,944: 2,347 / 2,392; torus 3,000, 43,104: 4,316 / 4,442).
+constexpr int kSplitSites = 8192;
 // Up to this many sites the emptiness pass takes each with four waves (ten
 // iterations at 1,296 tets / 131 sites 3.05 ms against 3.16 with one, at 48,000
 // / 2,000 3.75 against 3.79 for six; at 82,944 / 8,294 7.24 against 7.12).
@@ -150,6 +151,7 @@ int site_tcap_of(const vd_config& c) {
 
 struct vd_ctx {
   int device = 0;
+  int n_cus = 0;
   hipStream_t stream = nullptr;
   // second stream of the kNN step (the site queries beside the tet queries),
   // forked from and joined back into `stream` through the two events
@@ -499,7 +501,9 @@ int vd_ctx_create(vd_ctx** out, int device, const vd_config* cfg) {
     delete ctx;
     return VD_ERR_HIP;
   }
-  if (hipSetDevice(device) != hipSuccess || hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
+  if (hipSetDevice(device) != hipSuccess ||
+      hipDeviceGetAttribute(&ctx->n_cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess ||
+      hipStreamCreateWithFlags(&ctx->stream, hipStreamNonBlocking) != hipSuccess) {
     fprintf(stderr, "vd_ctx_create: cannot create a stream on device %d\n", device);
     delete ctx;
     return VD_ERR_HIP;
@@ -958,16 +962,12 @@ int vd_clip_step(vd_ctx* ctx) {
     const size_t list = (size_t)std::max(n_pairs, 1LL) * sizeof(unsigned);
     const bool cull = std::min(a.cull_depth, a.site_depth) > 0;
     bool two_lists = cull && n <= kFourWaveSites;
-    // the workgroups that stay resident (of more, the others find no unit left),
-    // for the records at the depth of moved sites, so that the second iteration
-    // needs no larger buffer than the first
-    vd::ClipArgs moved = a;
-    if (!wide) moved.site_depth = site_depth_of(c, ctx->K);
-    int resident = 0;
-    VD_HIP(vd::clip_site_blocks(moved, c.moments, c.accum, &resident), "clip");
-    const long long waves = std::min<long long>(blocks > 0 ? blocks : resident, resident);
-    if (blocks <= 0 && moved.site_depth == a.site_depth) blocks = resident;
-    if (blocks <= 0) VD_HIP(vd::clip_site_blocks(a, c.moments, c.accum, &blocks), "clip");
+    // the waves that hold record slots: those that stay resident (of more
+    // workgroups, the others find no unit left), at the depth of moved sites, so
+    // that the second iteration needs no larger buffer than the first
+    long long waves = (long long)ctx->n_cus *
+                      vd::clip_site_waves_per_cu(wide ? a.site_depth : site_depth_of(c, ctx->K), fast_tcap);
+    if (blocks > 0) waves = std::min<long long>(waves, blocks);
     // records: the estimate, plus the slots that the waves reserve ahead, a chunk
     // of each size class per wave.  The volume pass reads the unused ones too, so
     // the chunks are smaller where every wave has few pieces: us of four

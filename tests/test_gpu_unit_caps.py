@@ -17,7 +17,6 @@ pytestmark = pytest.mark.gpu
     (10, 2, 2, {"site_tcap": 12, "site_depth": 40}), (14, 8200, 64, {"site_tcap": 17, "site_depth": 16}),
     (14, 8200, 64, {"site_tcap": 17, "site_depth": 40, "clip_blocks": 5000}),
     (10, 600, 20, {"site_tcap": 17, "site_depth": 40, "moments": "reference"}),
-    (9, 2499, 64, {}), (9, 2500, 64, {}),  # the two sides of the units' size
     (24, 8294, 64, {}),  # 386,000 pieces: the automatic caps, at first for unmoved sites
 ])
 def test_units_at_small_caps(vdn, O, n, ns, tk, cfg):
