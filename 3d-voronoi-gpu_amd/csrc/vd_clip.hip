@@ -1692,8 +1692,9 @@ __global__ __launch_bounds__(64) void k_clip_site(ClipArgs a) {
 //
 // Testing each pair against the bisectors in list order was bound by VALU
 // issue: 335 instructions per 64 pairs and 545 us at 1M tets / 100,000 sites
-// (64M pairs); this takes 178 and 393 us.  The corners of the next 64 pairs are
-// loaded while these are tested (455 us without).
+// (64M pairs); this takes 212 and 404 us (191 and 392 with the limit's largest
+// coordinate over the whole mesh).  The corners of the next 64 pairs are loaded
+// while these are tested (455 us without).
 constexpr int kCullMaxDepth = 256;
 constexpr int kXcds = 8;  // MI355X: accelerator complex dies, one L2 each
 constexpr int kCullQueue = 128;

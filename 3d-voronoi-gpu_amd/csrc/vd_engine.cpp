@@ -74,8 +74,8 @@ constexpr double kWidePieces = 256e3;
 constexpr int kWideDepth = 96, kWideTcap = 32;
 // From this many sites on the clipping's work units are of 128 pairs, below it of
 // 64, which give every wave several.  Clipping us of four iterations, 64 against
-// 128: 8,294 sites (82,944 tets) 2,870 / 2,816, 13,171 (131,712) 3,660 / 3,530,
-// 16,000 (511,104) 6,340 / 6,010, 42,592 (511,104) 10,430 / 9,230; 600 sites (6,000)
+// 128: 8,294 sites (82,944 tets) 2,870 / 2,800, 13,171 (131,712) 3,660 / 3,520,
+// 16,000 (511,104) 6,315 / 5,990, 42,592 (511,104) 10,430 / 9,225; 600 sites (6,000)
 // 985 / 1,063, 1,500 (82,944) 1,566 / 1,617, 2,000 (48,000) 1,511 / 1,573.  Between
 // 2,500 and the line it is the survivors per site that decide, some 70 to 100 for
 // 128 (4,800 sites, 48,000 tets, 2,129 / 2,043: 64 leaves a small second unit), 150
@@ -972,8 +972,8 @@ int vd_clip_step(vd_ctx* ctx) {
     // of each size class per wave.  The volume pass reads the unused ones too, so
     // the chunks are smaller where every wave has few pieces: us of four
     // iterations, 64 against 128, 138k pieces 1,568 / 1,647, 169k 2,135 / 2,224,
-    // 223k 2,043 / 2,094; 294k 2,392 / 2,376, 386k 2,816 / 2,799, 2.4M 9,270 /
-    // 9,220.
+    // 223k 2,043 / 2,094; 294k 2,392 / 2,376, 386k 2,826 / 2,798, 2.4M 9,270 /
+    // 9,225.
     a.rec_chunk = pieces <= kWidePieces ? 64 : 128;
     const int stride = vd::rec_stride(fast_tcap);
     const long long ahead = 2LL * a.rec_chunk * std::min(waves, n_units);

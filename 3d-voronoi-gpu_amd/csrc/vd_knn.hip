@@ -707,8 +707,9 @@ constexpr int kQueryRun = VD_KNN_RUN, kQueryFill = VD_KNN_FILL;
 // and the registers to a fifth of a SIMD's.  kNN phase at 1M tets / 100,000
 // sites 1.55 -> 1.42 ms, 100,000 points and 1M random queries 2.14 -> 1.99 (M =
 // 1 with 192 or 320 points 1.44, M = 2 with 320 points 1.43, with 448 and 4
-// waves 1.49; 6 waves spill: 1.98).  Past k = 128 the list is longer, at the 3
-// waves that the registers allow.
+// waves 1.49; 6 waves, whose registers spill more than the 12 and 20 that they
+// do at 5, 1.98).  Past k = 128 the list is longer, at the 4 waves that its
+// registers and LDS allow (the bound asks for 3).
 template <int M>
 struct QueryShape {
   static constexpr int kUnionCap = M == 1 ? 256 : M == 2 ? 384 : 512;

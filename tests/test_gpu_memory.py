@@ -27,9 +27,11 @@ def _fill(hip, leave):
         p = ctypes.c_void_p()
         if _free(hip) < leave + size:
             size //= 2
-        else:
-            assert hip.L.hipMalloc(ctypes.byref(p), size) == 0
+        elif hip.L.hipMalloc(ctypes.byref(p), size) == 0:
             held.append(p)
+        else:  # (free, but not in one piece)
+            hip.L.hipGetLastError()
+            size //= 2
     return held
 
 
