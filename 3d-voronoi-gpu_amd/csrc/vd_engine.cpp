@@ -76,10 +76,11 @@ constexpr int kWideDepth = 96, kWideTcap = 32;
 // 64, which give every wave several.  Clipping us of four iterations, 64 against
 // 128: 8,294 sites (82,944 tets) 2,870 / 2,800, 13,171 (131,712) 3,660 / 3,520,
 // 16,000 (511,104) 6,315 / 5,990, 42,592 (511,104) 10,430 / 9,225; 600 sites (6,000)
-// 985 / 1,063, 1,500 (82,944) 1,566 / 1,617, 2,000 (48,000) 1,511 / 1,573.  Between
-// 2,500 and the line it is the survivors per site that decide, some 70 to 100 for
-// 128 (4,800 sites, 48,000 tets, 2,129 / 2,043: 64 leaves a small second unit), 150
-// for 64 (4,000, 82,944: 2,347 / 2,392; torus 3,000, 43,104: 4,316 / 4,442).
+// 985 / 1,063, 1,500 (82,944) 1,566 / 1,617, 2,000 (48,000) 1,511 / 1,573 (but 2,000
+// of 511,104 tets 3,455 / 3,374).  Between 2,500 and the line it is the survivors
+// per site that decide, some 70 to 100 for 128 (4,800 sites, 48,000 tets, 2,129 /
+// 2,043: 64 leaves a small second unit), 150 for 64 (4,000, 82,944: 2,347 / 2,392;
+// torus 3,000, 43,104: 4,316 / 4,442).
 constexpr int kSplitSites = 8192;
 // Up to this many sites the emptiness pass takes each with four waves (ten
 // iterations at 1,296 tets / 131 sites 3.05 ms against 3.16 with one, at 48,000
